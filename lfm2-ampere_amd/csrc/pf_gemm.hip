@@ -19,66 +19,117 @@
 // so does the reference's main loop.  Its nvcc build may contract the
 // epilogue's acc * scale + out into one fma, a difference of one rounding.
 //
-// MI355X design: workgroup = 128 weight rows x 128 tokens, 8 waves of 32
-// rows x 64 tokens, each a 1 x 2 pair of 32 x 32 v_mfma_i32_32x32x32_i8
-// tiles -- one 32-element Q4_0 block per MFMA, because the scales change from
-// block to block.  The 32-deep 32 x 32 form does four times the work of the
-// 16 x 16 one in about 2.2 times its issue time (15.4 against 7.1 ns per SIMD
-// on MI355X).  A operand: lane l supplies weight row l%32 of the tile,
-// elements 16(l/32)..+15, i.e. the low (l < 32) or high (l >= 32) nibbles of
-// the 16 bytes of the block (one shift, one mask per dword); B operand: the
-// same 16 elements of the activation row of token l%32.  The accumulator is
-// seeded with 0x4B400000 so the integer sum arrives as the float F.  Lane l's
-// 16 results of a tile are rows 8a + 4(l/32) + e (a, e = 0..3) of token l%32.
-// Staging, 4 blocks per stage in two LDS stages: weight and activation quants
-// by LDS DMA (no staging registers), the fp16 weight scales (each 32-row tile
-// permuted so that the 16 rows a lane needs are contiguous: two 16-byte
-// reads) and the (d8, 8 sum) token scales through registers; the next stage's
-// loads are issued right after the stage barrier and land during the compute.
-// 60 KB of LDS and at most 128 VGPRs: 2 workgroups, 4 waves per SIMD.
+// MI355X design: one 32-element Q4_0 block per MFMA, because the scales change
+// from block to block.  A wave covers MT weight rows x MT*NT tokens, MT = 32
+// (v_mfma_i32_32x32x32_i8) or 16 (16x16x32).  The accumulator is seeded with
+// 0x4B400000 so the integer sum arrives as the float F.  The row scale d4 of
+// the second fma is the same for every lane of a result row group: each lane
+// holds one row's d4 and the fma takes it by DPP (row_newbcast), so a block's
+// 16 row scales cost one LDS dword per lane and two blocks instead of 32
+// bytes per lane and block.
+// All operands reach LDS by LDS DMA (16 bytes per lane; the row scales 4), in
+// two stages of KC blocks, one barrier per stage.  A DMA instruction covers
+// whole runs of memory, a row's KC blocks side by side: with one row per lane
+// (64 cache lines per instruction) the address unit was the limit of every
+// launch under 4096 tokens.
+// What bounds it: the two fmas per output and block.  A step (one MFMA, its
+// 16 + 16 fmas, about 12 other VALU) measured 131 cycles per SIMD with 4
+// waves and everything in registers (v_fmac by DPP and v_fma_mix 4.3 cycles,
+// plain v_fma 2.7 as two waves issue together, the MFMA under them), 33 us
+// for 4096 tokens x 2048 x 2048; that launch takes 48.7-51.5 us (57-59 us in
+// the form before, whose d4 took 16 bytes more of LDS reads per lane and
+// block), about 7 of them the first stage's latency and the final stores of
+// 33.5 MB.  The blocks of an output are accumulated in order, so K cannot be
+// split: a launch of few tokens is a chain of bpr steps, and the shapes at the
+// launch below trade operand reuse for shorter chains.
 // Workgroups are mapped to tiles XCD by XCD (each XCD's L2 holds a few token
-// tiles' activations).  The output tile is written as float4 (4 consecutive
-// rows of one token).  Needs N % 128 == 0 and bpr % 8 == 0, as the
-// reference's pf_gemm_dense does (PF_BM = 128).
+// tiles' activations with every row tile).  The output tile is written as
+// float4 (4 consecutive rows of one token).  Needs N % 128 == 0 and bpr % 8
+// == 0, as the reference's pf_gemm_dense does (PF_BM = 128).
 #include "lk_common.h"
-
-#define PFG_BM 128                 // weight rows per workgroup
-#define PFG_BN 128                 // tokens per workgroup
-#define PFG_KC 4                   // blocks per LDS stage (the staging below moves exactly 4)
-#ifndef PFG_ABL
-#define PFG_ABL 0                  // measurement builds only: 1 no loads after stage 0, 2 no MFMA, 4 one add, 8 no store
-#endif
 
 typedef int lk_i4g __attribute__((ext_vector_type(4)));
 typedef int lk_i16g __attribute__((ext_vector_type(16)));
 typedef float lk_f16g __attribute__((ext_vector_type(16)));
 
-// One stage = 4 blocks.  a and b are filled by LDS DMA, 16 bytes per lane in
-// lane order, so their layouts are 16-byte slots: a[block][row] (the 16 quant
-// bytes of a weight block), b[block][half][token] (activation elements
-// 16*half .. +15 of a block).  The operand reads of 32 consecutive rows or
-// tokens are then 32 consecutive slots (conflict-free).
-struct alignas(16) PfgStage {
-    uint8_t  a[PFG_KC * PFG_BM * 16];        // 8 KB
-    int8_t   b[PFG_KC * 2 * PFG_BN * 16];    // 16 KB
-    _Float16 d[PFG_KC][PFG_BM];              // weight scales [block][row, permuted within 32-row tiles]
-    float2   s[PFG_BN][PFG_KC + 1];          // token scales (d8, 8 sum) [token][block]; the pad spreads 32 tokens over the banks
+// The shape of a launch: MT x MT MFMA tiles, NT of them along the tokens per
+// wave, WM x WN waves, KC blocks per stage.
+template <int MT_, int WM_, int WN_, int NT_, int KC_>
+struct PfgShape {
+    static constexpr int MT = MT_, WM = WM_, WN = WN_, NT = NT_, KC = KC_;
+    static constexpr int NW = WM * WN, BM = MT * WM, BN = MT * NT * WN;
+    // one stage in LDS, as 16-byte slots: a[row][block] (the 16 quant bytes of
+    // a weight block), b[token][2*block + half] (activation elements 16*half ..
+    // +15), s[token][block pair] (the (d8, 8 sum) of two blocks), then the
+    // dwords d[row][block pair] (two fp16 weight scales).  A row's blocks of a
+    // stage are contiguous here as in memory, so that a DMA instruction reads
+    // whole runs of 32 to 256 bytes.
+    static constexpr int OB = KC * BM * 16, OS = OB + KC * 2 * BN * 16, OD = OS + KC / 2 * BN * 16;
+    static constexpr int BYTES = OD + KC / 2 * BM * 4;
+    // DMA instructions per stage: a, b, s, d
+    static constexpr int NA = KC * BM / 64, NB = KC * 2 * BN / 64, NS = KC / 2 * BN / 64, ND = KC / 2 * BM / 64;
+    static constexpr int NI = NA + NB + NS + ND, PW = (NI + NW - 1) / NW;
+    static_assert(KC * BM % 64 == 0 && KC / 2 * BN % 64 == 0 && KC / 2 * BM % 64 == 0, "whole DMA instructions");
+    static_assert(8 % KC == 0, "a stage is whole for every accepted bpr");
 };
 
-// Position of row r (within a 32-row tile) in the permuted scale layout:
-// r = 8a + 4h + e  ->  16h + 4a + e, so lane half h finds its 16 rows
-// (a, e = 0..3) at 16h .. 16h+15.
-__device__ __forceinline__ int pfg_dperm(int r) {
-    return (r & ~31) | ((r & 4) << 2) | ((r >> 3 & 3) << 2) | (r & 3);
-}
+// Slot of piece x (0 .. n-1, n dividing 16) of a row of n slots: the pieces are
+// XOR-permuted within the row so that the same piece of 16 consecutive rows
+// lies in 16 different slots modulo 256 bytes (all LDS banks).  DMA writes
+// slots in lane order; the permutation is applied to its source addresses.
+__device__ __forceinline__ constexpr int pfg_slot(int n, int row, int x) { return row * n + (x ^ (row / (16 / n) % n)); }
 
-template <bool ADD>
-__global__ void __launch_bounds__(512, 4)
+// 4-byte LDS DMA (lane l's dword to lds + 4*l), wave-uniform base and per-lane offset.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void pfg_dma4(const void * sbase, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// acc[e] = fma(d4 of lane e of the 16-lane row, t[e], acc[e]) for 4 or 8 results from E0 on.
+// The s_nop covers the wait states between a VALU write of d and its DPP read,
+// which the compiler does not see inside the asm.
+#define PFG_FD(o, v, n) "v_fmac_f32_dpp %" #o ", %[d], %" #v " row_newbcast:%c" #n " row_mask:0xf bank_mask:0xf\n\t"
+template <int E0>
+__device__ __forceinline__ void pfg_fmac4(float * a, float d, const float * t) {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("s_nop 1\n\t" PFG_FD(0, 4, [e0]) PFG_FD(1, 5, [e1]) PFG_FD(2, 6, [e2]) PFG_FD(3, 7, [e3])
+        : "+v"(a[E0]), "+v"(a[E0 + 1]), "+v"(a[E0 + 2]), "+v"(a[E0 + 3])
+        : "v"(t[E0]), "v"(t[E0 + 1]), "v"(t[E0 + 2]), "v"(t[E0 + 3]), [d] "v"(d),
+          [e0] "n"(E0), [e1] "n"(E0 + 1), [e2] "n"(E0 + 2), [e3] "n"(E0 + 3));
+#endif
+}
+template <int E0>
+__device__ __forceinline__ void pfg_fmac8(float * a, float d, const float * t) {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("s_nop 1\n\t" PFG_FD(0, 8, [e0]) PFG_FD(1, 9, [e1]) PFG_FD(2, 10, [e2]) PFG_FD(3, 11, [e3])
+        PFG_FD(4, 12, [e4]) PFG_FD(5, 13, [e5]) PFG_FD(6, 14, [e6]) PFG_FD(7, 15, [e7])
+        : "+v"(a[E0]), "+v"(a[E0 + 1]), "+v"(a[E0 + 2]), "+v"(a[E0 + 3]),
+          "+v"(a[E0 + 4]), "+v"(a[E0 + 5]), "+v"(a[E0 + 6]), "+v"(a[E0 + 7])
+        : "v"(t[E0]), "v"(t[E0 + 1]), "v"(t[E0 + 2]), "v"(t[E0 + 3]),
+          "v"(t[E0 + 4]), "v"(t[E0 + 5]), "v"(t[E0 + 6]), "v"(t[E0 + 7]), [d] "v"(d),
+          [e0] "n"(E0), [e1] "n"(E0 + 1), [e2] "n"(E0 + 2), [e3] "n"(E0 + 3),
+          [e4] "n"(E0 + 4), [e5] "n"(E0 + 5), [e6] "n"(E0 + 6), [e7] "n"(E0 + 7));
+#endif
+}
+#undef PFG_FD
+
+// Bounded to the registers of 4 waves per SIMD although the LDS of the 128 x 64
+// shape admits 3: compiled for 3, its pipeline is ordered worse (4096 tokens
+// 51.5 -> 58.9 us).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Wpass-failed"
+template <class SH, bool ADD>
+__global__ void __launch_bounds__(64 * SH::NW, 4)
 lk_k_pf_gemm_q4_0(const uint8_t * __restrict__ qs, const _Float16 * __restrict__ d, int N, int bpr,
                   const int8_t * __restrict__ aqs, const float2 * __restrict__ asc, int ntok,
                   const float * __restrict__ scale, float * __restrict__ out, int out_ld) {
 #pragma clang fp contract(off)
-    __shared__ PfgStage stg[2];
+    constexpr int MT = SH::MT, NT = SH::NT, KC = SH::KC, NW = SH::NW, BM = SH::BM, BN = SH::BN, PW = SH::PW;
+    constexpr int NE = MT == 32 ? 16 : 4;              // results per lane and MFMA tile
+    __shared__ __attribute__((aligned(16))) uint8_t stg[2][SH::BYTES];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     // XCD-aware tile order: workgroups are dispatched round-robin over the 8
@@ -86,104 +137,155 @@ lk_k_pf_gemm_q4_0(const uint8_t * __restrict__ qs, const _Float16 * __restrict__
     // runs over the row tiles first: an XCD holds a few token tiles with all
     // row tiles, and its L2 fetches each activation row once instead of every
     // XCD fetching all of them.
-    const int nrt = N / PFG_BM, ntile = gridDim.x;
-    const int id = blockIdx.x;
-    const int L = (ntile % 8 == 0) ? (id % 8) * (ntile / 8) + id / 8 : id;
-    const int row0 = (L % nrt) * PFG_BM, tok0 = (L / nrt) * PFG_BN;
-    const int wr = (w & 3) * 32, wt = (w >> 2) * 64;   // the wave's 32 x 64 sub-tile
-    const int l32 = lane & 31, h = lane >> 5;
+    const int nrt = N / BM, ntile = gridDim.x;
+    const int id = blockIdx.x, x8 = id & 7, rem = ntile & 7;
+    const int L = x8 * (ntile >> 3) + (x8 < rem ? x8 : rem) + (id >> 3);
+    const int row0 = (L % nrt) * BM, tok0 = (L / nrt) * BN;
+    const int wr = (w % SH::WM) * MT, wt = (w / SH::WM) * (MT * NT);   // the wave's sub-tile
+    const int lm = lane & (MT - 1), h = lane / MT;     // MT 32: half 0/1; MT 16: lane group 0..3
     constexpr float MAGIC = 12582912.0f;               // 1.5 * 2^23 = float bits 0x4B400000
 
-    // ---- staging (4 blocks per stage).  LDS DMA: wave w brings block w/2 of
-    // weight rows 64(w%2) .. +63 (one instruction) and half w%2 of block w/2
-    // of all 128 tokens (two); through registers: for t < 128 the 4 fp16
-    // scales of weight row t, and block t%4 of token t/4's scale pair.
-    static_assert(PFG_KC == 4 && PFG_BM == 128 && PFG_BN == 128, "the staging assignment below");
-    const int sb = w >> 1, sh = w & 1;                 // this wave's DMA block and row half / token half
-    const uint32_t a_off = (uint32_t) ((64 * sh + lane) * bpr * 16 + 16 * sb);
-    uint32_t b_off[2];
+    // ---- staging: DMA instruction j = i*NW + w of a stage, i < PW, in the
+    // order a, b, s, d.  Its lanes' byte offsets from the stage's first block
+    // are formed once; a stage advances the uniform base only.
+    auto below = [&](int i, int n) -> bool {           // instruction i*NW + w < n; known at compile time unless the kinds meet in i
+        return i * NW + NW <= n || (i * NW < n && i * NW + w < n);
+    };
+    uint32_t voff[PW];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int t = tok0 + 64 * k + lane;
-        b_off[k] = (uint32_t) ((t < ntok ? t : ntok - 1) * bpr * 32 + 32 * sb + 16 * sh);   // clamped: in bounds
+    for (int i = 0; i < PW; ++i) {
+        const int j = i * NW + w;
+        if (below(i, SH::NA)) {
+            const int slot = 64 * j + lane, r = slot / KC;
+            voff[i] = (uint32_t) (r * bpr * 16 + (pfg_slot(KC, r, slot % KC) % KC) * 16);
+        } else if (below(i, SH::NA + SH::NB)) {
+            const int slot = 64 * (j - SH::NA) + lane, r = slot / (2 * KC), t = tok0 + r;
+            voff[i] = (uint32_t) (t < ntok ? t : ntok - 1) * (uint32_t) (bpr * 32)             // clamped: in bounds
+                      + (uint32_t) (pfg_slot(2 * KC, r, slot % (2 * KC)) % (2 * KC) * 16);
+        } else if (below(i, SH::NA + SH::NB + SH::NS)) {
+            const int slot = 64 * (j - SH::NA - SH::NB) + lane, r = slot / (KC / 2), t = tok0 + r;
+            voff[i] = (uint32_t) (t < ntok ? t : ntok - 1) * (uint32_t) (bpr * 8)
+                      + (uint32_t) (pfg_slot(KC / 2, r, slot % (KC / 2)) % (KC / 2) * 16);
+        } else {
+            const int slot = 64 * (j - SH::NA - SH::NB - SH::NS) + lane, r = slot / (KC / 2);
+            voff[i] = (uint32_t) (r * bpr * 2 + slot % (KC / 2) * 4);
+        }
     }
     const uint8_t * a_base = qs + (size_t) row0 * bpr * 16;
-    const int bt = tid >> 2, bq = tid & 3;
-    const int stok = (tok0 + bt < ntok) ? tok0 + bt : ntok - 1;
-    const _Float16 * gd = d + (size_t) (row0 + (tid & 127)) * bpr;                    // + kb0 (tid < 128)
-    const float2 * gs = asc + (size_t) stok * bpr + bq;                               // + kb0
-    const int dp = pfg_dperm(tid & 127);
-    uint2 rs, rd = make_uint2(0, 0);
-    auto fetch = [&](int kb0, PfgStage & S) {
-        lk_dma16c_so(a_base + 16 * kb0, a_off, lk_lds_addr(S.a + (sb * PFG_BM + 64 * sh) * 16));
+    const _Float16 * d_base = d + (size_t) row0 * bpr;
+    const uint32_t lds0 = lk_lds_addr(&stg[0][0]);
+    auto fetch = [&](int ck) {
+        const uint32_t sb = lds0 + (uint32_t) ((ck & 1) * SH::BYTES);
+        const int kb0 = ck * KC;
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-            lk_dma16c_so(aqs + 32 * kb0, b_off[k], lk_lds_addr(S.b + ((2 * sb + sh) * PFG_BN + 64 * k) * 16));
-        if (tid < 128) rd = *(const uint2 *) (gd + kb0);
-        rs = *(const uint2 *) (gs + kb0);
-    };
-    auto stash = [&](PfgStage & S) {
-        if (tid < 128) {
-            S.d[0][dp] = __builtin_bit_cast(_Float16, (unsigned short) (rd.x & 0xffff));
-            S.d[1][dp] = __builtin_bit_cast(_Float16, (unsigned short) (rd.x >> 16));
-            S.d[2][dp] = __builtin_bit_cast(_Float16, (unsigned short) (rd.y & 0xffff));
-            S.d[3][dp] = __builtin_bit_cast(_Float16, (unsigned short) (rd.y >> 16));
+        for (int i = 0; i < PW; ++i) {
+            const int j = i * NW + w;                  // wave-uniform
+            if (below(i, SH::NA)) lk_dma16c_so(a_base + 16 * kb0, voff[i], sb + (uint32_t) (1024 * j));
+            else if (below(i, SH::NA + SH::NB)) lk_dma16c_so(aqs + 32 * kb0, voff[i], sb + (uint32_t) (SH::OB + 1024 * (j - SH::NA)));
+            else if (below(i, SH::NA + SH::NB + SH::NS))
+                lk_dma16c_so(asc + kb0, voff[i], sb + (uint32_t) (SH::OS + 1024 * (j - SH::NA - SH::NB)));
+            else if (below(i, SH::NI)) pfg_dma4(d_base + kb0, voff[i], sb + (uint32_t) (SH::OD + 256 * (j - SH::NA - SH::NB - SH::NS)));
         }
-        S.s[bt][bq] = make_float2(__uint_as_float(rs.x), __uint_as_float(rs.y));
     };
 
     const int mb = 0x4B400000;
-    const lk_i16g seed = { mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb };
-    const int nsh = 4 * h;                             // low or high nibbles
-    lk_f16g acc[2];
+    // the row whose d4 this lane holds: result e of the lane's row group, e = lane % 16 (MT 16: % 4)
+    const int c16 = lane & 15;
+    const int drow = wr + (MT == 32 ? 8 * (c16 >> 2) + 4 * h + (c16 & 3) : 4 * h + (c16 & 3));
+    float acc[NT][NE];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
+        for (int e = 0; e < NE; ++e) acc[j][e] = 0.0f;
 
-    // One barrier per stage: the DMA into stage (ck+1)&1 is issued after the
-    // barrier of stage ck, which every wave reaches only when done reading
-    // stage ck-1 (the same buffer); the register-staged scales of stage ck go
-    // into a buffer last read at ck-2.
-    const int nck = bpr / PFG_KC;
-    fetch(0, stg[0]);
+    // The DMA of stage ck + 1 is issued after the barrier of stage ck, which
+    // every wave reaches only when done reading stage ck - 1 (the same buffer).
+    // (Rings of three and four stages were slower: their LDS costs co-resident
+    // workgroups, 640 tokens 14.9 -> 18.6 and 21.1 us.)
+    const int nck = bpr / KC;
+    fetch(0);
     for (int ck = 0; ck < nck; ++ck) {
-        PfgStage & S = stg[ck & 1];
-        lk_wait_vm<0>();                               // this wave's DMA and scale loads of stage ck
-        stash(S);
+        lk_wait_vm<0>();
         __syncthreads();
-        if (ck + 1 < nck && !((PFG_ABL & 1) && ck > 0)) fetch((ck + 1) * PFG_KC, stg[(ck + 1) & 1]);
+        if (ck + 1 < nck) fetch(ck + 1);
+        const uint8_t * S = stg[ck & 1];
+        // The stage's NI = KC*NT MFMAs in the order block, token tile, as a
+        // pipeline: operands are read two steps ahead and the MFMA of step
+        // i + 1 is issued before the fmas of step i, so that it runs under
+        // them (the sched_barriers keep only MFMAs from moving).
+        constexpr int NI = KC * NT;
+        lk_i4g av[2], bv[2];                           // operands of the step's block / step, by parity
+        uint32_t d2[2];
+        float4 sv[2][NT];
+        lk_f16g F[2];
+        auto load = [&](int i) {
+            const int b = i / NT, j = i % NT;
+            if (j == 0) {
+                if (b % 2 == 0) {
+                    d2[(b / 2) & 1] = *(const uint32_t *) (S + SH::OD + (drow * (KC / 2) + b / 2) * 4);
 #pragma unroll
-        for (int b = 0; b < PFG_KC; ++b) {
-            const uint4 q = *(const uint4 *) (S.a + (b * PFG_BM + wr + l32) * 16);
-            const lk_i4g a = { (int) ((q.x >> nsh) & 0x0F0F0F0Fu), (int) ((q.y >> nsh) & 0x0F0F0F0Fu),
-                               (int) ((q.z >> nsh) & 0x0F0F0F0Fu), (int) ((q.w >> nsh) & 0x0F0F0F0Fu) };
-            // d4 of this lane's 16 rows of the row tile (fp16, two 16-byte reads)
-            const lk_h8 d4lo = *(const lk_h8 *) &S.d[b][wr + 16 * h];
-            const lk_h8 d4hi = *(const lk_h8 *) &S.d[b][wr + 16 * h + 8];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const lk_i4g bv = *(const lk_i4g *) (S.b + ((2 * b + h) * PFG_BN + wt + 32 * j + l32) * 16);
-                const lk_f16g F = (PFG_ABL & 2) ? __builtin_bit_cast(lk_f16g, (lk_i16g){ a[0], a[1], a[2], a[3], bv[0], bv[1], bv[2], bv[3], a[0], a[1], a[2], a[3], bv[0], bv[1], bv[2], bv[3] })
-                                                : __builtin_bit_cast(lk_f16g, __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bv, seed, 0, 0, 0));
-                const float2 sv = S.s[wt + 32 * j + l32][b];
-                const float c = __builtin_fmaf(sv.x, MAGIC, sv.y);
-#pragma unroll
-                for (int e = 0; e < 16; ++e)           // result e = row 8(e/4) + 4h + e%4 = scale slot e
-                    acc[j][e] = (PFG_ABL & 4) ? acc[j][e] + F[e] :
-                                __builtin_fmaf((float) (e < 8 ? d4lo[e] : d4hi[e - 8]),
-                                               __builtin_fmaf(sv.x, F[e], -c), acc[j][e]);
+                    for (int jj = 0; jj < NT; ++jj)
+                        sv[(b / 2) & 1][jj] = *(const float4 *) (S + SH::OS + pfg_slot(KC / 2, wt + MT * jj + lm, b / 2) * 16);
+                }
+                const uint8_t * ap = S + pfg_slot(KC, wr + lm, b) * 16;
+                if constexpr (MT == 32) av[b & 1] = *(const lk_i4g *) ap;
+                else { const int2 q = *(const int2 *) (ap + 8 * (h & 1)); av[b & 1] = (lk_i4g){ q.x, q.y, 0, 0 }; }
             }
+            const uint8_t * bp = S + SH::OB + pfg_slot(2 * KC, wt + MT * j + lm, 2 * b + (MT == 32 ? h : h >> 1)) * 16;
+            if constexpr (MT == 32) bv[i & 1] = *(const lk_i4g *) bp;
+            else { const int2 q = *(const int2 *) (bp + 8 * (h & 1)); bv[i & 1] = (lk_i4g){ q.x, q.y, 0, 0 }; }
+        };
+        lk_i4g a;                                      // nibbles of the block, low or high by lane half
+        auto mfma = [&](int i) {
+            const int b = i / NT;
+            if (i % NT == 0) {
+                const int nsh = MT == 32 ? 4 * h : 4 * (h >> 1);
+#pragma unroll
+                for (int k = 0; k < (MT == 32 ? 4 : 2); ++k) a[k] = (int) (((uint32_t) av[b & 1][k] >> nsh) & 0x0F0F0F0Fu);
+            }
+            if constexpr (MT == 32) {
+                const lk_i16g seed = { mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb, mb };
+                F[i & 1] = __builtin_bit_cast(lk_f16g, __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bv[i & 1], seed, 0, 0, 0));
+            } else {
+                const lk_i4g seed = { mb, mb, mb, mb };
+                const int2 a2 = make_int2(a[0], a[1]), b2 = make_int2(bv[i & 1][0], bv[i & 1][1]);
+                const lk_f4 f = __builtin_bit_cast(lk_f4, __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                    __builtin_bit_cast(long, a2), __builtin_bit_cast(long, b2), seed, 0, 0, 0));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) F[i & 1][e] = f[e];
+            }
+        };
+        load(0);
+        if (NI > 1) load(1);
+        mfma(0);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int b = i / NT, j = i % NT, u = b & 1;
+            // the scales of this step, before load(i + 2) may replace them
+            const uint32_t dd = d2[(b / 2) & 1];
+            const float4 ss = sv[(b / 2) & 1][j];
+            __builtin_amdgcn_sched_barrier(0x7F7);
+            if (i + 1 < NI) mfma(i + 1);
+            __builtin_amdgcn_sched_barrier(0x7F7);
+            if (i + 2 < NI) load(i + 2);
+            const float d4 = (float) __builtin_bit_cast(_Float16, (unsigned short) (u ? dd >> 16 : dd & 0xffff));
+            const float d8 = u ? ss.z : ss.x, s8 = u ? ss.w : ss.y;
+            const float c = __builtin_fmaf(d8, MAGIC, s8);
+            float t[NE];
+#pragma unroll
+            for (int e = 0; e < NE; ++e) t[e] = __builtin_fmaf(d8, F[i & 1][e], -c);   // row 8(e/4) + 4h + e%4
+            if constexpr (MT == 32) { pfg_fmac8<0>(acc[j], d4, t); pfg_fmac8<8>(acc[j], d4, t); }
+            else pfg_fmac4<0>(acc[j], d4, t);
         }
     }
-    // epilogue: lane holds rows 8a + 4h .. +3 of the row tile for token l32 of each token tile
+    // epilogue: lane holds, per token tile, 4 consecutive rows NE/4 times
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int t = tok0 + wt + 32 * j + l32;
+    for (int j = 0; j < NT; ++j) {
+        const int t = tok0 + wt + MT * j + lm;
         if (t >= ntok) continue;
         const float sc = scale ? scale[t] : 1.0f;
 #pragma unroll
-        for (int a4 = 0; a4 < 4; ++a4) {
+        for (int a4 = 0; a4 < NE / 4; ++a4) {
             float4 * p = (float4 *) (out + (size_t) t * out_ld + row0 + wr + 8 * a4 + 4 * h);
             float4 v = make_float4(acc[j][4 * a4] * sc, acc[j][4 * a4 + 1] * sc,
                                    acc[j][4 * a4 + 2] * sc, acc[j][4 * a4 + 3] * sc);
@@ -191,9 +293,20 @@ lk_k_pf_gemm_q4_0(const uint8_t * __restrict__ qs, const _Float16 * __restrict__
                 const float4 o = *p;
                 v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
             }
-            if (!(PFG_ABL & 8) || v.x == 1234.5f) *p = v;
+            *p = v;
         }
     }
+}
+#pragma clang diagnostic pop
+
+template <class SH>
+static void pfg_launch(const uint8_t * qs, const _Float16 * d, int N, int bpr, const int8_t * aqs, const float2 * asc,
+                       int ntok, const float * scale, float * out, int out_ld, int add, hipStream_t st) {
+    const dim3 grid((N / SH::BM) * ((ntok + SH::BN - 1) / SH::BN));
+    if (add)
+        hipLaunchKernelGGL((lk_k_pf_gemm_q4_0<SH, true>), grid, dim3(64 * SH::NW), 0, st, qs, d, N, bpr, aqs, asc, ntok, scale, out, out_ld);
+    else
+        hipLaunchKernelGGL((lk_k_pf_gemm_q4_0<SH, false>), grid, dim3(64 * SH::NW), 0, st, qs, d, N, bpr, aqs, asc, ntok, scale, out, out_ld);
 }
 
 extern "C" int lk_pf_gemm_q4_0(const void * qs, const void * d, int N, int bpr, const int8_t * aqs,
@@ -202,9 +315,9 @@ extern "C" int lk_pf_gemm_q4_0(const void * qs, const void * d, int N, int bpr, 
     if (N < 0 || ntok < 0 || bpr < 1)
         return lk_fail(hipErrorInvalidValue, "lk_pf_gemm_q4_0: N %d / ntok %d / bpr %d", N, ntok, bpr);
     if (N == 0 || ntok == 0) return 0;
-    if (N % PFG_BM != 0 || bpr % 8 != 0 || out_ld % 4 != 0 || out_ld < N)
+    if (N % 128 != 0 || bpr % 8 != 0 || out_ld % 4 != 0 || out_ld < N)
         return lk_fail(hipErrorInvalidValue, "lk_pf_gemm_q4_0: N %d must be a multiple of %d, bpr %d of %d, out_ld %d a multiple of 4 and >= N",
-                       N, PFG_BM, bpr, 8, out_ld);
+                       N, 128, bpr, 8, out_ld);
     // the kernel addresses activation rows with 32-bit byte offsets
     if ((size_t) ntok * bpr * 32 > 0xFFFFFFFFull)
         return lk_fail(hipErrorInvalidValue, "lk_pf_gemm_q4_0: ntok %d x bpr %d activations exceed 4 GiB", ntok, bpr);
@@ -214,13 +327,26 @@ extern "C" int lk_pf_gemm_q4_0(const void * qs, const void * d, int N, int bpr, 
     if (((uintptr_t) qs & 15) || ((uintptr_t) d & 7) || ((uintptr_t) aqs & 15) || ((uintptr_t) asc & 15) ||
         ((uintptr_t) out & 15) || ((uintptr_t) scale & 3))
         return lk_fail(hipErrorInvalidValue, "lk_pf_gemm_q4_0: misaligned argument (qs, aqs, asc, out 16 B; d 8 B; scale 4 B)");
-    const dim3 grid((N / PFG_BM) * ((ntok + PFG_BN - 1) / PFG_BN));
     const hipStream_t st = lk_stream(stream);
-    if (add)
-        hipLaunchKernelGGL(lk_k_pf_gemm_q4_0<true>, grid, dim3(512), 0, st, (const uint8_t *) qs, (const _Float16 *) d,
-                           N, bpr, aqs, (const float2 *) asc, ntok, scale, out, out_ld);
-    else
-        hipLaunchKernelGGL(lk_k_pf_gemm_q4_0<false>, grid, dim3(512), 0, st, (const uint8_t *) qs, (const _Float16 *) d,
-                           N, bpr, aqs, (const float2 *) asc, ntok, scale, out, out_ld);
+    auto go = [&](auto sh) {
+        pfg_launch<decltype(sh)>((const uint8_t *) qs, (const _Float16 *) d, N, bpr, aqs, (const float2 *) asc, ntok,
+                                 scale, out, out_ld, add, st);
+    };
+    // The shape (2048 x 2048 weights, us per launch in a hipGraph; old: the one
+    // shape of 128 x 128 in 8 waves with whole-line-per-lane staging that
+    // served every size before):
+    //   tokens             1    77   201   333   640  1100  1536  2048  2999  4096
+    //   old             26.4  27.8  29.7  30.9  32.2  32.6  33.3  34.7  50.7  58.9
+    //   32 x 32          6.6   7.0   8.9  11.8  16.5  27.0  32.8  41.1  57.6  75.2
+    //   128 x 128       21.6  22.5  23.5  23.3  24.1  25.8  26.6  27.7  47.6  53.5
+    //   128 x 64        16.8  17.8  18.6  18.7  19.3  27.8  27.6  29.1  40.5  51.6
+    // A launch takes a whole chain of bpr blocks per round of workgroups.  Up
+    // to 7 tiles of 32 x 32 per CU the shortest chain wins; then 128 x 128 in
+    // 16 waves while one round of the chip holds all of its tiles; past that
+    // 128 x 64, three workgroups per CU, whose rounds end less ragged.
+    const long t32 = (long) (N / 32) * ((ntok + 31) / 32), t128 = (long) (N / 128) * ((ntok + 127) / 128);
+    if (t32 <= 7 * 256)    go(PfgShape<16, 2, 2, 1, 8>{});
+    else if (t128 <= 256)  go(PfgShape<32, 4, 4, 1, 4>{});
+    else                   go(PfgShape<32, 4, 1, 2, 4>{});
     return lk_launch_status("lk_pf_gemm_q4_0");
 }

@@ -85,3 +85,30 @@ def test_attention_output_chain(lk, oracle):
     ref = o @ w.reshape(2048, 2048).T
     delta = got[rows].astype(np.float64) - x0[rows]
     assert np.max(np.abs(delta - ref)) / np.max(np.abs(ref)) < 5e-2
+
+
+# The three workgroup shapes meet at 1792 tiles of 32 x 32 and at 256 tiles of
+# 128 x 128 (N, bpr, ntok): both sides of each line, token counts off every
+# tile, one and several stages.
+EDGES = [(2048, 8, 896), (2048, 8, 897), (2048, 16, 2048), (2048, 8, 2049), (3072, 16, 1409), (128, 8, 33),
+         (128, 24, 31), (3072, 8, 597)]
+
+
+@pytest.mark.parametrize("N,bpr,ntok", EDGES, ids=[f"N{a}_b{b}_t{c}" for a, b, c in EDGES])
+@pytest.mark.parametrize("add", [False, True])
+def test_pf_gemm_shapes_bit_exact(lk, oracle, N, bpr, ntok, add):
+    rng = np.random.default_rng(N + 7 * bpr + ntok)
+    qs, d = _weights(rng, N, bpr)
+    aqs, asc = oracle.pf_quant_rows(rng.standard_normal((ntok, bpr * 32)).astype(np.float32), ntok, bpr * 32, bpr)
+    out0 = rng.standard_normal((ntok, N)).astype(np.float32)
+    scale = rng.uniform(0.5, 2.0, ntok).astype(np.float32) if add else None
+    # the weight scales at an address that is a multiple of 8 bytes only
+    dd = torch.empty(N * bpr + 4, dtype=torch.int16, device="cuda")[4:]
+    dd.copy_(dev(d.reshape(-1).view(np.int16)))
+    out = dev(out0)
+    note(f"pf gemm q4_0 shapes N={N} bpr={bpr} ntok={ntok} add={add}")
+    lk.pf_gemm_q4_0(dev(qs.reshape(-1)), dd, N, bpr, dev(aqs.reshape(-1)), dev(asc.reshape(-1)), ntok, out, N, add,
+                    None if scale is None else dev(scale))
+    torch.cuda.synchronize()
+    want = oracle.pf_gemm_q4_0(qs, d, N, bpr, aqs, asc, ntok, scale=scale, out=out0, add=add)
+    assert np.array_equal(host(out).view(np.uint32), want.view(np.uint32))
