@@ -97,22 +97,72 @@ lk_k_pf_k8(const _Float16 * __restrict__ kc, int p0, int p1, const float * __res
 // reference's (prefill.cu:1304-1318): 16 strided fp32 running sums (p = g,
 // g+16, ...), then those 16 added in index order, then / n -- kept identical
 // so the smoothing vector matches the reference bit for bit.
-__global__ void __launch_bounds__(1024)
+//
+// The 16 x 512 running sums are serial chains of n/16 adds; what a launch can
+// choose is how their values arrive.  Workgroup (head, 8 dims), 64 of them,
+// heads spread over the XCDs so that the workgroups that share a cache line
+// share an L2: 8 waves bring tiles of 1024 rows x 16 bytes by LDS DMA, three
+// tiles in flight, and 128 threads walk one chain each out of LDS.  Against
+// one workgroup per head whose threads load their own values (8 workgroups, a
+// memory round trip per few adds), in a hipGraph, rows read before: 1000 rows
+// 8.5 -> 5.2 us, 2999 21.5 -> 7.1, 8192 54.9 -> 9.1, 32768 593 -> 40; right
+// behind the producer that wrote 2999 rows 55 -> 6 us.
+#define KM_ROWS 1024
+#define KM_NBUF 4
+template <bool ALIGNED>                                   // kc a multiple of 16 bytes (else plain 2-byte loads)
+__global__ void __launch_bounds__(512)
 lk_k_pf_kmean(const _Float16 * __restrict__ kc, int n, float * __restrict__ cm) {
 #pragma clang fp contract(off)
-    __shared__ float part[16][LK_HEAD_DIM];
-    const int h = blockIdx.x, d = threadIdx.x & 63, g = threadIdx.x >> 6;
+    __shared__ __attribute__((aligned(16))) _Float16 s_t[KM_NBUF][KM_ROWS][8];
+    __shared__ float part[16][8];
+    const int h = blockIdx.x % LK_N_KV_HEADS, dg = blockIdx.x / LK_N_KV_HEADS;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const _Float16 * src = kc + h * LK_HEAD_DIM + 8 * dg;
+    constexpr int PW = KM_ROWS / 64 / 8;                  // DMA instructions per wave and tile
+    const int nt = (n + KM_ROWS - 1) / KM_ROWS;
+    auto fetch = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < PW; ++i) {
+            const int r = 64 * (PW * w + i);
+            const int p = t * KM_ROWS + r + lane;
+            const _Float16 * row = src + (size_t) (p < n ? p : n - 1) * LK_KV_ROW;
+            if constexpr (ALIGNED) lk_dma16c(row, lk_lds_addr(&s_t[t % KM_NBUF][r][0]));
+            else
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s_t[t % KM_NBUF][r + lane][e] = row[e];
+        }
+    };
+    for (int t = 0; t < KM_NBUF - 1 && t < nt; ++t) fetch(t);
+    const int d = tid & 7, g = tid >> 3;                  // chain of threads 0..127
     float s = 0.0f;
-    for (int p = g; p < n; p += 16) s += (float) kc[((size_t) p * LK_N_KV_HEADS + h) * LK_HEAD_DIM + d];
-    part[g][d] = s;
+    for (int t = 0; t < nt; ++t) {
+        const int later = nt - 1 - t;                     // tiles issued after t, at most KM_NBUF - 2
+        if (later >= 2)      lk_wait_vm<2 * PW>();
+        else if (later == 1) lk_wait_vm<PW>();
+        else                 lk_wait_vm<0>();
+        __syncthreads();                                  // everyone's rows; tile t - 1 consumed
+        if (t + KM_NBUF - 1 < nt) fetch(t + KM_NBUF - 1);
+        if (tid < 128) {
+            const _Float16 (*T)[8] = s_t[t % KM_NBUF];
+            const int rows = n - t * KM_ROWS;
+            if (rows >= KM_ROWS) {
+#pragma unroll 16
+                for (int r = 0; r < KM_ROWS; r += 16) s += (float) T[r + g][d];
+            } else {
+                for (int r = g; r < rows; r += 16) s += (float) T[r][d];
+            }
+        }
+    }
+    if (tid < 128) part[g][d] = s;
     __syncthreads();
-    if (g == 0) {
+    if (tid < 8) {
         float t = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) t += part[i][d];
-        cm[h * LK_HEAD_DIM + d] = t / (float) n;
+        for (int i = 0; i < 16; ++i) t += part[i][tid];
+        cm[h * LK_HEAD_DIM + 8 * dg + tid] = t / (float) n;
     }
 }
+static_assert(KM_NBUF == 4, "the waits of lk_k_pf_kmean");
 
 // ---------------------------------------------------------------------------
 // Flash attention.
@@ -1246,8 +1296,12 @@ extern "C" int lk_pf_k8(const void * kc, int p0, int p1, const float * cm, int k
 extern "C" int lk_pf_kmean(const void * kc, int n, float * cm, void * stream) {
     if (n <= 0) return lk_fail(hipErrorInvalidValue, "lk_pf_kmean: n must be > 0");
     if (!kc || !cm) return lk_fail(hipErrorInvalidValue, "lk_pf_kmean: null pointer argument");
-    hipLaunchKernelGGL(lk_k_pf_kmean, dim3(LK_N_KV_HEADS), dim3(1024), 0, lk_stream(stream),
-                       (const _Float16 *) kc, n, cm);
+    if ((uintptr_t) kc & 15)
+        hipLaunchKernelGGL(lk_k_pf_kmean<false>, dim3(LK_N_KV_HEADS * 8), dim3(512), 0, lk_stream(stream),
+                           (const _Float16 *) kc, n, cm);
+    else
+        hipLaunchKernelGGL(lk_k_pf_kmean<true>, dim3(LK_N_KV_HEADS * 8), dim3(512), 0, lk_stream(stream),
+                           (const _Float16 *) kc, n, cm);
     return lk_launch_status("lk_pf_kmean");
 }
 
