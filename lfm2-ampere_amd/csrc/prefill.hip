@@ -1063,6 +1063,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
 #pragma unroll
             for (int qb = 0; qb < PF_QB; ++qb) {
                 const int row = 16 * qb + col;
+                if (qbase + row >= m) continue;           // never merged
 #pragma unroll
                 for (int db = 0; db < 4; ++db) A[(4 * db + g) * PF_BQ + row] = acc[db][qb];
                 if (g == 0) ML[row] = make_float2(moff(qb), acc[4][qb][0]);
@@ -1134,35 +1135,45 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
     }
 }
 
-// Merge of the parts of split query blocks: workgroup (split block, kv head,
-// half of the dims), thread = (head, row) over 32 dims -- one Q8_1 block; the
-// parts are weighted 2^(m_p - M) with the exact max M and summed in part
-// order.  All of a thread's loads are independent, so it waits for memory
-// about twice.
-__global__ void __launch_bounds__(256)
+// Merge of the parts of split query blocks: a thread holds (head, row) over 32
+// dims -- one Q8_1 block; the parts are weighted 2^(m_p - M) with the exact max
+// M and summed in a fixed order.  Bound by memory latency: a thread's loads of
+// up to MAXP parts are independent, one round trip per pass.
+//   NPG 1: workgroup (split block, kv head, half of the dims), threads (head,
+//          row), four parts per pass.
+//   NPG 8: one workgroup per head as well, threads (part group, row): group g
+//          sums parts g, g + 8, ..., two per pass, and the 8 sums are merged
+//          through LDS in group order.  For launches of more than 8 parts per
+//          block, a short chunk deep in a prompt: 77 rows at position 30011
+//          (37 parts) 29.6 -> 11.2 us, 5 rows at 30000 (64 parts) 52.3 -> 10.7,
+//          300 at 9000 (15) 12.9 -> 10.4; with 4 to 5 parts its LDS pass
+//          loses (1100 rows at 3333 11.7 -> 16.5, 1500 at 0 10.6 -> 16.1).
+#define PF_CMB_LD 36                                      // floats per (group, row) in LDS: 32 dims, m, l, pad
+template <int NPG>
+__global__ void __launch_bounds__(NPG == 1 ? 256 : 64 * NPG)
 lk_k_pf_combine(const float * __restrict__ pbuf, int m, int P, const PfWork work, float * __restrict__ o,
                 int8_t * __restrict__ aqs, float2 * __restrict__ asc) {
 #pragma clang fp contract(off)
-    constexpr int MAXP = 4;                               // parts merged per pass
-    const int kvh = blockIdx.y, hb = blockIdx.z;          // dims 32hb .. 32hb+31
+    const int kvh = blockIdx.y, hb = blockIdx.z & 1;      // dims 32hb .. 32hb+31
     const int qt = work.split_qt[blockIdx.x];
-    const int np = work.nparts[qt];
     const int slot = work.slot0[qt];
-    const int row = threadIdx.x & 63, h = threadIdx.x >> 6;
+    const int row = threadIdx.x & 63, h = NPG == 1 ? threadIdx.x >> 6 : blockIdx.z >> 1;
+    const int pg = NPG == 1 ? 0 : threadIdx.x >> 6;
     const int qr = qt * PF_BQ + row;
-    if (qr >= m) return;
+    if (NPG == 1 && qr >= m) return;
+    const int np = qr < m ? work.nparts[qt] : 0;          // rows past m hold nothing
     auto base = [&](int p) { return pbuf + (size_t) ((slot + p) * LK_N_KV_HEADS + kvh) * PF_PART_SLOT; };
     float M = -INFINITY, L = 0.0f;
     lk_f4 A[8] = {};
-    // one pass over parts [p0, p0 + W): all loads first (one memory round
-    // trip), then the merge in part order
+    // one pass over parts p0, p0 + NPG, ... (W of them): all loads first (one
+    // memory round trip), then the merge in part order
     auto pass = [&](auto wc, int p0) {
         constexpr int W = decltype(wc)::value;
         float2 ml[W];
         lk_f4 a[W][8];
 #pragma unroll
         for (int i = 0; i < W; ++i) {
-            const int p = (p0 + i < np) ? p0 + i : p0;    // clamped: loads stay in bounds
+            const int p = (p0 + i * NPG < np) ? p0 + i * NPG : p0;   // clamped: loads stay in bounds
             ml[i] = ((const float2 *) (base(p) + PF_PART_ACC))[h * PF_BQ + row];
             const lk_f4 * src = (const lk_f4 *) base(p) + (size_t) (h * 16 + 8 * hb) * PF_BQ + row;
 #pragma unroll
@@ -1170,14 +1181,14 @@ lk_k_pf_combine(const float * __restrict__ pbuf, int m, int P, const PfWork work
         }
         float Mn = M;
 #pragma unroll
-        for (int i = 0; i < W; ++i) if (p0 + i < np) Mn = fmaxf(Mn, ml[i].x);
+        for (int i = 0; i < W; ++i) if (p0 + i * NPG < np) Mn = fmaxf(Mn, ml[i].x);
         const float r = lk_exp2(M - Mn);                  // 0 on the first pass (M = -inf)
         L *= r;
 #pragma unroll
         for (int c = 0; c < 8; ++c) A[c] *= r;
 #pragma unroll
         for (int i = 0; i < W; ++i) {
-            if (p0 + i >= np) break;
+            if (p0 + i * NPG >= np) break;
             const float wgt = lk_exp2(ml[i].x - Mn);
             L += ml[i].y * wgt;
 #pragma unroll
@@ -1185,9 +1196,35 @@ lk_k_pf_combine(const float * __restrict__ pbuf, int m, int P, const PfWork work
         }
         M = Mn;
     };
-    // two parts per block is the common case: no redundant loads for it
-    if (np == 2) pass(std::integral_constant<int, 2>{}, 0);
-    else for (int p0 = 0; p0 < np; p0 += MAXP) pass(std::integral_constant<int, MAXP>{}, p0);
+    if constexpr (NPG == 1) {
+        // two parts per block is the common case: no redundant loads for it
+        if (np == 2) pass(std::integral_constant<int, 2>{}, 0);
+        else for (int p0 = 0; p0 < np; p0 += 4) pass(std::integral_constant<int, 4>{}, p0);
+    } else {
+        for (int p0 = pg; p0 < np; p0 += 2 * NPG) pass(std::integral_constant<int, 2>{}, p0);
+        // (a group without parts holds M = -inf, L = 0, A = 0: weight 0 below)
+        __shared__ __attribute__((aligned(16))) float s_g[NPG][PF_BQ][PF_CMB_LD];
+        float * G = s_g[pg][row];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) *(lk_f4 *) (G + 4 * c) = A[c];
+        *(float2 *) (G + 32) = make_float2(M, L);
+        __syncthreads();
+        if (pg != 0 || qr >= m) return;
+#pragma unroll
+        for (int g = 1; g < NPG; ++g) M = fmaxf(M, s_g[g][row][32]);
+        L = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) A[c] = (lk_f4){ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int g = 0; g < NPG; ++g) {
+            const float * E = s_g[g][row];
+            const float2 ml = *(const float2 *) (E + 32);
+            const float wgt = lk_exp2(ml.x - M);
+            L += ml.y * wgt;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) A[c] += *(const lk_f4 *) (E + 4 * c) * wgt;
+        }
+    }
     const float il = 1.0f / L;
     float x[32];
 #pragma unroll
@@ -1663,8 +1700,14 @@ static int pf_attn_launch(const int8_t * q8, const float * qsc, const float * qc
                        q8, qsc, qcs, qh, m, P, k8, ksc, kstride, kc, vc, near, sink, o, aqs, asc, wk, pbuf);
     int rc = lk_launch_status(what);
     if (rc) return rc;
-    hipLaunchKernelGGL(lk_k_pf_combine, dim3(wk.n_split, LK_N_KV_HEADS, 2), dim3(256), 0, st,
-                       (const float *) pbuf, m, P, wk, o, aqs, asc);
+    int npmax = 0;
+    for (int i = 0; i < wk.n_split; ++i) npmax = std::max(npmax, (int) wk.nparts[wk.split_qt[i]]);
+    if (npmax <= 8)
+        hipLaunchKernelGGL(lk_k_pf_combine<1>, dim3(wk.n_split, LK_N_KV_HEADS, 2), dim3(256), 0, st,
+                           (const float *) pbuf, m, P, wk, o, aqs, asc);
+    else
+        hipLaunchKernelGGL(lk_k_pf_combine<8>, dim3(wk.n_split, LK_N_KV_HEADS, 2 * LK_G), dim3(512), 0, st,
+                           (const float *) pbuf, m, P, wk, o, aqs, asc);
     rc = lk_launch_status(what);
     if (rc) return rc;
     return work ? 0 : pf_part_release(st, dev);      // a caller's workspace is ordered by the caller

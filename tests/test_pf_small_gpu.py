@@ -1,6 +1,6 @@
 """The small kernels around the prefill attention at the sizes where their tiles
 end, against the oracle, bit for bit: the K smoothing mean and the standalone
-planar Q8_1."""
+planar Q8_1; and the merge of many split-K parts."""
 import numpy as np
 import pytest
 import torch
@@ -49,3 +49,36 @@ def test_quant_rows_bit_exact(lk, oracle, rows, kb, pad, offset):
     wq, ws = oracle.pf_quant_rows(X, rows, ld, kb)
     assert np.array_equal(host(qs), np.asarray(wq).reshape(rows, kb * 32))
     assert np.array_equal(host(sc).view(np.uint32), np.asarray(ws, np.float32).reshape(rows, kb, 2).view(np.uint32))
+
+
+# more than 8 parts per block take the part-group merge: part counts off its 8
+# groups of two, ragged last blocks, both outputs.  2e-3 of the largest output
+# is the bound every prefill case here is held to: p rounded to fp16 (2^-11
+# each) on rows of a few thousand keys.
+@pytest.mark.parametrize("m,P,tiles", [(1, 640, 1), (5, 2100, 2), (77, 1500, 1), (130, 3000, 3), (64, 4000, 1)])
+def test_combine_many_parts(lk, oracle, m, P, tiles):
+    from gpu_util import dev_h
+    K, V, Q = oracle.mt_prefill_case(99 + m, m, P, 0.0, False)
+    kc, vc, qh = dev_h(K), dev_h(V), dev_h(Q)
+    try:
+        lk.pf_split_override(tiles)
+        items = lk.pf_plan_items(m, P, 0, 0, False)
+        assert max(sum(1 for i in items if i[0] == q) for q in {i[0] for i in items}) > 8
+        outs = []
+        note(f"pf_attn many parts m={m} P={P} tiles={tiles}")
+        for _ in range(2):
+            o = torch.full((m, 2048), float("nan"), device="cuda")
+            aqs = torch.zeros(m, 2048, dtype=torch.int8, device="cuda")
+            asc = torch.zeros(m, 64, 2, device="cuda")
+            lk.pf_attn_q81(qh, m, P, kc, vc, o, aqs, asc)
+            torch.cuda.synchronize()
+            outs.append((host(o), host(aqs), host(asc)))
+    finally:
+        lk.pf_split_override(0)
+    for a, b in zip(*outs):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), "run-to-run bit-identical"
+    rows = np.array(sorted({0, m // 2, m - 1}), np.int32)
+    ref = oracle.pf_ref(Q, m, P, K, V, rows=rows)
+    assert oracle.rel_err(outs[0][0][rows], ref[rows]) <= 2e-3
+    q, sc = oracle.pf_quant_rows(outs[0][0], m, 2048, 64)
+    assert np.array_equal(outs[0][1], q) and np.array_equal(outs[0][2].view(np.uint32), sc.view(np.uint32))
