@@ -99,3 +99,22 @@ def test_override(lk_host):
 def test_bad_arguments(lk_host):
     with pytest.raises(Exception):
         lk_host.pf_plan_items(0, 0, 0, 0, True)
+
+
+# chunks of few blocks are cut into equal pieces: block counts on both sides of
+# the rule's lines, key ranges from less than a piece to more than 64 of them,
+# all exact, mixed and almost all int8
+@pytest.mark.parametrize("m", [1, 5, 64, 77, 512, 513, 700, 768, 769])
+@pytest.mark.parametrize("P", [0, 63, 130, 3000, 30011, 130000])
+@pytest.mark.parametrize("near,sink,int8", [(1024, 1, True), (64, 0, True), (1 << 20, 1, True), (0, 0, False)])
+def test_few_blocks(lk_host, m, P, near, sink, int8):
+    items = lk_host.pf_plan_items(m, P, near, sink, int8)
+    if not items:
+        return
+    by_block = check_plan(items, m, P, near, sink, int8)
+    nq = len(by_block)
+    if nq <= 8 or (nq <= 12 and P >= m):
+        for qt, pieces in by_block.items():
+            # equal cost but for whole tiles, and for the diagonal tile that no piece may start past
+            c = [cost(qt, lo, hi, P, near, sink, int8) for lo, hi, _ in sorted(pieces)]
+            assert max(c) - min(c[:-1], default=c[-1]) <= 3 * 1.4
