@@ -108,3 +108,24 @@ def test_untracked_loads_untouched_until_their_wait(tmp_path):
         assert loads == (20 if fused else 4), (name, loads)
         # D = 3 tiles of RPW = 4 rows per wave stay in flight
         assert first_wait == 12, (name, first_wait)
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_untracked_loads_with_the_makefiles_own_flags(tmp_path):
+    """The same on the command line the Makefile builds decode.hip with
+    (kernel-argument preload included), whatever its flags become."""
+    cmd = next(l for l in subprocess.run(["make", "-n", "-B", "_build/decode.hip.o"], cwd=PKG, check=True,
+                                         capture_output=True, text=True).stdout.split("\n") if " -c -x hip " in l)
+    args = cmd.split(" 2>&1")[0].replace("-c -x hip", "--offload-device-only -S -x hip").split()
+    asm = tmp_path / "decode.s"
+    args[args.index("-o") + 1] = str(asm)
+    subprocess.run(args, check=True, cwd=PKG, capture_output=True)
+    txt = asm.read_text()
+    assert "kernarg_preload_length" in txt
+    for fused in (0, 1):
+        name = "_Z15lk_k_attn_splitILb%dE" % fused
+        i = txt.index("\n" + name) + 1
+        body = [l.strip() for l in txt[i:txt.index(".Lfunc_end", i)].split("\n")]
+        loads, first_wait = _check_paths(name, body)
+        assert loads == (20 if fused else 4), (name, loads)
+        assert first_wait == 12, (name, first_wait)
