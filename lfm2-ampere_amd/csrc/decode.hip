@@ -172,8 +172,8 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     }
 
     // ---- fetch: wave w brings rows w, w+8, ... of each tile (K rows first) ----
-    const char * kg = (const char *) kc + 16 * lane;
-    const char * vg = (const char *) vc + 16 * lane;
+    const char * kg = (const char *) kc;
+    const char * vg = (const char *) vc;
     const uint32_t lds0 = lk_lds_addr(&s_tile[0][0]);
     // first position of the slice's tile it
     auto tile_pos = [&](int it) -> int { return (sp + ns * it) * LK_DEC_TILE; };
@@ -181,6 +181,10 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     auto fetch = [&](int it) {
         const uint32_t base = lds0 + (uint32_t) ((it % LK_DEC_NBUF) * LK_DEC_TILEB);
         const int p0 = tile_pos(it);
+        // a tile past the slice's last is read by no one: every lane of its
+        // DMAs takes the same 16 bytes (one line a row instead of a whole row;
+        // up to 4096 positions at least two of a slice's first three tiles)
+        const uint32_t lo = it < ntile ? 16u * (uint32_t) lane : 0u;
 #pragma unroll
         for (int i = 0; i < RPW; ++i) {
             const int row = w + 8 * i;                         // 0 .. 2*TILE-1
@@ -192,7 +196,7 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
             // fetch on one L2 channel), all tiles of an empty slice row 0;
             // they are masked or land in buffers no tile of the slice uses
             const size_t o = (size_t) (it < ntile && tp < seq ? tp : clamp_row) * (LK_KV_ROW * 2);
-            lk_dma16((isv ? vg : kg) + o, base + (uint32_t) (row * LK_DEC_ROWB));
+            lk_dma16((isv ? vg : kg) + o + lo, base + (uint32_t) (row * LK_DEC_ROWB));
         }
     };
     // Wait until tile `it` is resident for the whole workgroup.  When tile it
