@@ -68,8 +68,10 @@ __device__ __forceinline__ void lk_split_h(float x, _Float16 & hi, _Float16 & lo
 // ^32, ^16: lk_xrow_sum adds in that order, both partners the same two
 // values), then 4, 2, 1 in lane; 1/sqrt in fp64 rounded once; the rotation of
 // the pair (d, d+32) with the table entry d.
-__device__ __forceinline__ void lk_norm_rope_pair8(float (&lo)[8], float (&hi)[8], const float (&wlo)[8],
-                                                   const float (&whi)[8], int g, const float * s_c, const float * s_s) {
+// The norm and the rotation are separate steps: the norm needs no angle, so it
+// stands before the barrier behind which the table is complete.
+__device__ __forceinline__ void lk_norm_pair8(float (&lo)[8], float (&hi)[8], const float (&wlo)[8],
+                                              const float (&whi)[8]) {
 #pragma clang fp contract(off)
     float t[8];
 #pragma unroll
@@ -82,10 +84,14 @@ __device__ __forceinline__ void lk_norm_rope_pair8(float (&lo)[8], float (&hi)[8
     const float arg = ss * (1.0f / LK_HEAD_DIM) + LK_EPS_F;
     const float inv = (float) (1.0 / sqrt((double) arg));
 #pragma unroll
+    for (int i = 0; i < 8; ++i) { lo[i] = (lo[i] * inv) * wlo[i]; hi[i] = (hi[i] * inv) * whi[i]; }
+}
+__device__ __forceinline__ void lk_rope_pair8(float (&lo)[8], float (&hi)[8], int g, const float * s_c, const float * s_s) {
+#pragma clang fp contract(off)
+#pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int d = 8 * g + i;
-        const float yl = (lo[i] * inv) * wlo[i], yh = (hi[i] * inv) * whi[i];
-        const float c = s_c[d], sn = s_s[d];
+        const float yl = lo[i], yh = hi[i], c = s_c[d], sn = s_s[d];
         lo[i] = yl * c - yh * sn;
         hi[i] = yl * sn + yh * c;
     }
@@ -148,7 +154,14 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     // Slice sp holds tiles T = sp + ns * it, it < ntile, of the nt tiles that
     // cover [0, seq): slices differ by at most one tile.
     const int nt = (seq + LK_DEC_TILE - 1) / LK_DEC_TILE;
-    const int ntile = (sp < ns && sp < nt) ? (nt - sp + ns - 1) / ns : 0;
+    // (with a target of one tile per slice more tiles than slices means that
+    // the slice count is the cap, a constant: no division on the way to the
+    // first DMA)
+    int ntile;
+    if constexpr (LK_ATTN_TARGET_N <= LK_DEC_TILE)
+        ntile = sp < nt ? (nt - sp + LK_ATTN_SPLIT - 1) / LK_ATTN_SPLIT : 0;
+    else
+        ntile = (sp < ns && sp < nt) ? (nt - sp + ns - 1) / ns : 0;
     // A slice with no tiles (ntile = 0: sp >= nt or sp >= ns) takes the same
     // path with an empty tile loop, so its record is the neutral one (m =
     // -inf, l = 0, acc = 0) and every slot the combine reads is valid without
@@ -157,7 +170,7 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     // be free to reuse their registers (a store address formed in one of
     // them would be overwritten by the arriving data).
     const int pos = seq - 1;
-    const bool own_pos = FUSED && (nt - 1) % ns == sp;     // this slice holds position pos (its last tile)
+    const bool own_pos = FUSED && ntile > 0 && sp + ns * (ntile - 1) == nt - 1;   // this slice holds position pos (its last tile)
     if constexpr (FUSED) {          // loaded by every workgroup: see the wait below
         const float * kp = pr.k_src + w * LK_HEAD_DIM + 8 * g;
         const float * vp = pr.v_src + w * LK_HEAD_DIM + 8 * g;
@@ -226,6 +239,19 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     // after it only in straight-line code.
 #pragma unroll
     for (int i = 0; i < D; ++i) fetch(i);
+    __shared__ float s_c[FUSED ? LK_HEAD_DIM / 2 : 1], s_s[FUSED ? LK_HEAD_DIM / 2 : 1];
+    if constexpr (FUSED) {
+        // The 32 (cos, sin) entries of position seq-1, 4 per wave, under the
+        // latency of the loads; every lane forms and writes entry 4w +
+        // (lane & 3), so that there is no branch of ours while they are
+        // pending.  With the side-by-side norms below, per layer of the step
+        // graph 10.73 -> 10.04 us at 20 positions, 11.19 -> 10.90 at 2500,
+        // 18.93 -> 18.81 at 32768.
+        float c, sn;
+        lk_rope_angle(pos, rfreq, c, sn);
+        s_c[4 * w + (lane & 3)] = c;
+        s_s[4 * w + (lane & 3)] = sn;
+    }
     lk_wait_vm_tie<D * RPW>(qv);
     if constexpr (FUSED) {
         lk_wait_vm_tie<D * RPW>(qwv);
@@ -243,34 +269,35 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
         unpack(kv4, klo, khi); unpack(vv4, vlo, vhi); unpack(kwv, kwlo, kwhi);
     }
 
-    // Folded producer: the 32 (cos, sin) entries of position seq-1, 4 per wave.
-    __shared__ float s_c[FUSED ? LK_HEAD_DIM / 2 : 1], s_s[FUSED ? LK_HEAD_DIM / 2 : 1];
+    // Folded producer: q and the new row's k normalised and rotated side by side
+    // in every workgroup (each a chain of about 400 ns; the new row's workgroup,
+    // on the step's critical path, would otherwise run them one after the other).
     lk_h8 kv_h[4];                                         // its K lo, K hi, V lo, V hi (fp16)
     if constexpr (FUSED) {
-        if (lane < 4) lk_rope_angle(pos, rfreq, s_c[4 * w + lane], s_s[4 * w + lane]);
+        lk_norm_pair8(qlo, qhi, qwlo, qwhi);
+        lk_norm_pair8(klo, khi, kwlo, kwhi);
         __syncthreads();
-        if (own_pos) {
-            float lo[8], hi[8];
+        lk_rope_pair8(qlo, qhi, g, s_c, s_s);
+        lk_rope_pair8(klo, khi, g, s_c, s_s);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) { lo[i] = klo[i]; hi[i] = khi[i]; }
-            lk_norm_rope_pair8(lo, hi, kwlo, kwhi, g, s_c, s_s);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                kv_h[0][i] = (_Float16) lo[i]; kv_h[1][i] = (_Float16) hi[i];
-                kv_h[2][i] = (_Float16) vlo[i]; kv_h[3][i] = (_Float16) vhi[i];
-            }
-            if (col == 0) {
-                const size_t off = ((size_t) pos * LK_N_KV_HEADS + w) * LK_HEAD_DIM + 8 * g;
-                _Float16 * kw = (_Float16 *) kc, * vw = (_Float16 *) vc;
-                *(lk_h8 *) (kw + off) = kv_h[0]; *(lk_h8 *) (kw + off + 32) = kv_h[1];
-                *(lk_h8 *) (vw + off) = kv_h[2]; *(lk_h8 *) (vw + off + 32) = kv_h[3];
-                float * ko = pr.k_out + w * LK_HEAD_DIM + 8 * g;
-                *(lk_f4 *) ko        = (lk_f4){ lo[0], lo[1], lo[2], lo[3] };
-                *(lk_f4 *) (ko + 4)  = (lk_f4){ lo[4], lo[5], lo[6], lo[7] };
-                *(lk_f4 *) (ko + 32) = (lk_f4){ hi[0], hi[1], hi[2], hi[3] };
-                *(lk_f4 *) (ko + 36) = (lk_f4){ hi[4], hi[5], hi[6], hi[7] };
-            }
+        for (int i = 0; i < 8; ++i) {
+            kv_h[0][i] = (_Float16) klo[i]; kv_h[1][i] = (_Float16) khi[i];
+            kv_h[2][i] = (_Float16) vlo[i]; kv_h[3][i] = (_Float16) vhi[i];
         }
+        auto put64 = [&](float * o, const float (&lo)[8], const float (&hi)[8]) {
+            *(lk_f4 *) o        = (lk_f4){ lo[0], lo[1], lo[2], lo[3] };
+            *(lk_f4 *) (o + 4)  = (lk_f4){ lo[4], lo[5], lo[6], lo[7] };
+            *(lk_f4 *) (o + 32) = (lk_f4){ hi[0], hi[1], hi[2], hi[3] };
+            *(lk_f4 *) (o + 36) = (lk_f4){ hi[4], hi[5], hi[6], hi[7] };
+        };
+        if (own_pos && col == 0) {
+            const size_t off = ((size_t) pos * LK_N_KV_HEADS + w) * LK_HEAD_DIM + 8 * g;
+            _Float16 * kw = (_Float16 *) kc, * vw = (_Float16 *) vc;
+            *(lk_h8 *) (kw + off) = kv_h[0]; *(lk_h8 *) (kw + off + 32) = kv_h[1];
+            *(lk_h8 *) (vw + off) = kv_h[2]; *(lk_h8 *) (vw + off + 32) = kv_h[3];
+            put64(pr.k_out + w * LK_HEAD_DIM + 8 * g, klo, khi);
+        }
+        if (sp == 0 && col < 4) put64(pr.q_out + qrow, qlo, qhi);   // the working q, once
     }
 
     // Scores are computed transposed, S^T = K . Q^T (v_mfma_f32_16x16x32_f16):
@@ -286,16 +313,6 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
         float lo[8], hi[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) { lo[i] = qlo[i]; hi[i] = qhi[i]; }
-        if constexpr (FUSED) {
-            lk_norm_rope_pair8(lo, hi, qwlo, qwhi, g, s_c, s_s);
-            if (sp == 0 && col < 4) {                       // the working q, once
-                float * qo = pr.q_out + qrow;
-                *(lk_f4 *) qo        = (lk_f4){ lo[0], lo[1], lo[2], lo[3] };
-                *(lk_f4 *) (qo + 4)  = (lk_f4){ lo[4], lo[5], lo[6], lo[7] };
-                *(lk_f4 *) (qo + 32) = (lk_f4){ hi[0], hi[1], hi[2], hi[3] };
-                *(lk_f4 *) (qo + 36) = (lk_f4){ hi[4], hi[5], hi[6], hi[7] };
-            }
-        }
         // The fp16 hi half of q must be finite: a head whose largest |q| reaches
         // 2^15 is scaled by 2^-k first (exact) so that it stays below 2^15, and
         // its scores are scaled back by 2^k below.  k = 0 for every other head
