@@ -368,7 +368,19 @@ __device__ __forceinline__ void lk_pf_q81_epilogue(const lk_f4 (&a)[4], bool sto
 // barriers of their own (a counter in LDS), not at the workgroup barrier, so
 // the two waves of a SIMD (one per group) drift into different phases of
 // their tiles, as two unpaired workgroups do.
-template <bool INT8, bool PAIR, bool Q81>
+//
+// SHORT (unpaired): a last block of at most 32 (16) rows runs a tile loop of its
+// own with two (one) of its four 16-query blocks; the others hold no rows.  Such
+// a tile costs about 0.65 (0.55) of a whole one -- barrier, key scales and
+// operand reads stay -- and the workgroup beside it on the CU takes what it
+// leaves, so the plan keeps its cuts and every result its bits.  Attention and
+// merge, whole tiles -> this: 5 rows at 30000 int8 36.8 -> 26.7 us, 20 at 60000
+// 50.4 -> 37.6, 32 at 9000 22.6 -> 18.9, 77 at 30011 (Q8_1) 65.9 -> 55.7, fp16
+// 64.4 -> 51.0, 400 at 9000 (Q8_1) 71.7 -> 62.5, fp16 1100 at 3333 72.3 -> 64.3;
+// from 980 rows at 0 to 2060 at 4000 within 1% of it.  One loop with a
+// branch per pair of query blocks spilled (44-60 bytes a lane); the loops are
+// separate for that.
+template <bool INT8, bool PAIR, bool Q81, bool SHORT = false>
 __global__ void __launch_bounds__(PAIR ? 512 : 256, PAIR ? 1 : 2)
 lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
              const float * __restrict__ qcs, const _Float16 * __restrict__ qh, int m, int P,
@@ -759,7 +771,9 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
     // ---- one 64-key tile.  Mode and mask are wave-uniform run-time branches:
     // bodies specialised per mode (one loop each, or one loop with a branch to
     // each) measured 40% slower, the register allocator then spilled.
-    auto tile = [&](const PfStage & S, int kt) {
+    auto tile = [&](const PfStage & S, int kt, auto nblk) {
+        constexpr int NB = decltype(nblk)::value;          // 16-query blocks with rows in them: 1, 2 or 4
+        constexpr int NJ = NB == 1 ? 1 : 2;                // of them at a time
         const int md = mode_of(kt);
         const bool msk = mask_of(kt);
         const int kb0 = kt * PF_BK;
@@ -787,7 +801,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
         // Two query blocks at a time (scores of 64 keys x 32 queries in flight);
         // in a mixed tile the first pair is exact, the second int8.
 #pragma unroll
-        for (int hq = 0; hq < 2; ++hq) {
+        for (int hq = 0; hq < NB / NJ; ++hq) {
             const bool ex = (md == PF_EXACT) || (md == PF_MIXED && hq == 0);
             // x: unpaired launches, the score in units of 1/sq; PAIR, the
             // exponent argument x*sq - moff itself (one fma per score on exact
@@ -799,11 +813,11 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                 __builtin_amdgcn_readfirstlane(__float_as_int(mst[2 * hq])) == __float_as_int(-INFINITY);
             float mo2[2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) mo2[j] = first ? 0.0f : mst[2 * hq + j];
+            for (int j = 0; j < NJ; ++j) mo2[j] = first ? 0.0f : mst[2 * hq + j];
             if (ex) {
                 lk_h8 qa[2][2];
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
+                for (int j = 0; j < NJ; ++j) {
                     const int8_t * qrow = s_q[qw] + o_q + 16 * PF_Q_LD * (2 * hq + j);
                     qa[j][0] = *(const lk_h8 *) qrow;
                     qa[j][1] = *(const lk_h8 *) (qrow + 64);
@@ -824,7 +838,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                     const lk_h8 k0 = PAIR ? kf[kb][0] : *(const lk_h8 *) (S.kh + o_kh0 + 2048 * kb);
                     const lk_h8 k1 = PAIR ? kf[kb][1] : *(const lk_h8 *) (S.kh + o_kh1 + 2048 * kb);
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         const int qb = 2 * hq + j;
                         lk_f4 c = { 0.f, 0.f, 0.f, 0.f };
                         c = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qa[j][0], c, 0, 0, 0);
@@ -842,7 +856,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         const lk_f4 c = lk_mfma_qk8_magic(ka[kb], qf8[2 * hq + j]);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
@@ -853,7 +867,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
             }
             if (msk) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
+                for (int j = 0; j < NJ; ++j) {
                     // key kb0+16kb+4g+i is masked iff 16kb+i > qpos - kb0 - 4g
                     const int dq = P + qbase + 16 * (2 * hq + j) + col - kb0 - 4 * g;
 #pragma unroll
@@ -871,7 +885,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
             // reduction.
             auto make_p = [&]() {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
+                for (int j = 0; j < NJ; ++j) {
                     const int qb = 2 * hq + j;
                     if constexpr (PAIR) {
 #pragma unroll
@@ -907,7 +921,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                 // finite), and the arguments taken against it
                 if (first) {
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         const float mn = row_max(j) + PF_P_BIAS;
                         mst[2 * hq + j] = mn;
 #pragma unroll
@@ -932,7 +946,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
             __builtin_amdgcn_sched_barrier(0);
             unsigned pw[16];
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int kk = 0; kk < 2; ++kk) {
                     const lk_i4 uw = __builtin_bit_cast(lk_i4, pb[2 * hq + j][kk]);
@@ -940,7 +954,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                     for (int e = 0; e < 4; ++e) pw[8 * j + 4 * kk + e] = (unsigned) uw[e];
                 }
 #pragma unroll
-            for (int n = 16; n > 1; n = (n + 2) / 3)                // OR tree, three words per op
+            for (int n = 8 * NJ; n > 1; n = (n + 2) / 3)                // OR tree, three words per op
 #pragma unroll
                 for (int t = 0; t < (n + 2) / 3; ++t)
                     pw[t] = pw[3 * t] | (3 * t + 1 < n ? pw[3 * t + 1] : 0u) | (3 * t + 2 < n ? pw[3 * t + 2] : 0u);
@@ -950,14 +964,16 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                 // p words against 0x7800.
                 lk_u16x8 pm = __builtin_elementwise_max(__builtin_bit_cast(lk_u16x8, pb[2 * hq][0]),
                                                         __builtin_bit_cast(lk_u16x8, pb[2 * hq][1]));
-                pm = __builtin_elementwise_max(pm, __builtin_bit_cast(lk_u16x8, pb[2 * hq + 1][0]));
-                pm = __builtin_elementwise_max(pm, __builtin_bit_cast(lk_u16x8, pb[2 * hq + 1][1]));
+                if constexpr (NJ == 2) {
+                    pm = __builtin_elementwise_max(pm, __builtin_bit_cast(lk_u16x8, pb[2 * hq + 1][0]));
+                    pm = __builtin_elementwise_max(pm, __builtin_bit_cast(lk_u16x8, pb[2 * hq + 1][1]));
+                }
                 const lk_u16x4 p4 = __builtin_elementwise_max(pm.s0123, pm.s4567);
                 const lk_u16x2 p2 = __builtin_elementwise_max(p4.s01, p4.s23);
                 const unsigned short p1 = p2.x > p2.y ? p2.x : p2.y;
                 if (__ballot(p1 >= 0x7800u)) {                 // wave-uniform, rare
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         const int qb = 2 * hq + j;
                         if constexpr (PAIR) {
                             // the offset of the queries past the limit moves up
@@ -1013,11 +1029,11 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                 const lk_h4 hi = lk_ds_tr4(S.v + o_vd[db] + 4096 * kk + 2048);   // keys +16
                 const lk_h8 va = { lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3] };
 #pragma unroll
-                for (int qb = 0; qb < PF_QB; ++qb)
+                for (int qb = 0; qb < NB; ++qb)
                     acc[db][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[qb][kk], acc[db][qb], 0, 0, 0);
             }
 #pragma unroll
-            for (int qb = 0; qb < PF_QB; ++qb)
+            for (int qb = 0; qb < NB; ++qb)
                 acc[4][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb[qb][kk], acc[4][qb], 0, 0, 0);
         }
     };
@@ -1049,12 +1065,17 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
 
     if constexpr (!PAIR) {
         // ---- tile loop: one barrier per tile; tile kt+1 streams in while kt computes
-        for (int kt = kt_lo; kt < kt_hi; ++kt) {
-            lk_wait_vm<0>();                              // this wave's part of tile kt landed
-            __syncthreads();                              // ... everyone's; tile kt-1 fully consumed
-            if (kt + 1 < kt_hi) issue(kt + 1);            // into the stage tile kt-1 used
-            tile(st[kt & 1], kt);
-        }
+        auto tiles = [&](auto nblk) {
+            for (int kt = kt_lo; kt < kt_hi; ++kt) {
+                lk_wait_vm<0>();                          // this wave's part of tile kt landed
+                __syncthreads();                          // ... everyone's; tile kt-1 fully consumed
+                if (kt + 1 < kt_hi) issue(kt + 1);        // into the stage tile kt-1 used
+                tile(st[kt & 1], kt, nblk);
+            }
+        };
+        if (SHORT && m - qbase <= 16) tiles(std::integral_constant<int, 1>{});
+        else if (SHORT && m - qbase <= 32) tiles(std::integral_constant<int, 2>{});
+        else tiles(std::integral_constant<int, PF_QB>{});
 
         if (pslot >= 0) {                                 // a part: unnormalised partial
             float * R = pbuf + (size_t) (pslot * LK_N_KV_HEADS + kvh) * PF_PART_SLOT;
@@ -1078,7 +1099,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
             lk_wait_vm<0>();
             gsync();
             if (it + 1 < g_ns) issue_step(it + 1);
-            tile(st[2 * grp + (it & 1)], g_tile(it));
+            tile(st[2 * grp + (it & 1)], g_tile(it), std::integral_constant<int, PF_QB>{});
             if (grp == 0 && it == nki - 1) {
                 // bi is complete: write it; group A goes on with bj, whose fp16
                 // Q block group B's wave of the same head holds in LDS
@@ -1768,8 +1789,12 @@ static int pf_attn_launch(const int8_t * q8, const float * qsc, const float * qc
     // gives coarser pieces, none at all an unsplit launch); without one the
     // library's static scratch is used
     pf_plan(m, P, near, sink, INT8, Q81, split_override, work ? work_bytes / sizeof(float) : (size_t) PF_PART_CAP, wk);
+    const int nq = (m + PF_BQ - 1) / PF_BQ, last = m - (nq - 1) * PF_BQ;
+    // at most 32 rows in the last block: the kernel that skips its empty query
+    // blocks (from 33 rows on there is nothing it could skip)
+    auto * kernel = last <= PF_BQ / 2 ? lk_k_pf_attn<INT8, false, Q81, true> : lk_k_pf_attn<INT8, false, Q81, false>;
     if (wk.n_items == 0) {
-        hipLaunchKernelGGL((lk_k_pf_attn<INT8, false, Q81>), dim3((m + PF_BQ - 1) / PF_BQ, LK_N_KV_HEADS), dim3(256), 0, st,
+        hipLaunchKernelGGL(kernel, dim3(nq, LK_N_KV_HEADS), dim3(256), 0, st,
                            q8, qsc, qcs, qh, m, P, k8, ksc, kstride, kc, vc, near, sink, o, aqs, asc, wk,
                            (float *) nullptr);
         return lk_launch_status(what);
@@ -1781,7 +1806,7 @@ static int pf_attn_launch(const int8_t * q8, const float * qsc, const float * qc
     int err = 0, dev = 0;
     float * pbuf = work ? work : pf_part_acquire(st, err, dev);
     if (!pbuf) return err;
-    hipLaunchKernelGGL((lk_k_pf_attn<INT8, false, Q81>), dim3(wk.n_items * LK_N_KV_HEADS), dim3(256), 0, st,
+    hipLaunchKernelGGL(kernel, dim3(wk.n_items * LK_N_KV_HEADS), dim3(256), 0, st,
                        q8, qsc, qcs, qh, m, P, k8, ksc, kstride, kc, vc, near, sink, o, aqs, asc, wk, pbuf);
     int rc = lk_launch_status(what);
     if (rc) return rc;

@@ -82,3 +82,53 @@ def test_combine_many_parts(lk, oracle, m, P, tiles):
     assert oracle.rel_err(outs[0][0][rows], ref[rows]) <= 2e-3
     q, sc = oracle.pf_quant_rows(outs[0][0], m, 2048, 64)
     assert np.array_equal(outs[0][1], q) and np.array_equal(outs[0][2].view(np.uint32), sc.view(np.uint32))
+
+
+# A last block of at most 16 or 32 rows runs only the query blocks that hold
+# rows.  The same rows inside a chunk of whole blocks go through the full tile:
+# the same key tiles in the same order (unsplit), so every output is the same
+# bits.  The chunk's further queries are zero, as the kernel takes rows that are
+# not there: a query whose weights pass 2^15 makes its wave raise every running
+# maximum whose weights passed 2^14, so other neighbours could move a rounding.
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 65, 80, 81, 96, 97])
+@pytest.mark.parametrize("P,near,sink", [(0, 1024, 1), (700, 64, 1), (1999, 128, 0)])
+@pytest.mark.parametrize("int8", [True, False])
+def test_short_last_block_is_bit_identical(lk, m, P, near, sink, int8):
+    full = (m + 63) // 64 * 64
+    S, ks = P + full, lk.kstride_for(P + full)
+    g = torch.Generator(device="cuda").manual_seed(m + P)
+    qh = (torch.randn(full, 2048, device="cuda", generator=g) / 4).half()
+    qh[m:] = 0
+    kc = torch.randn(S, 512, device="cuda", generator=g).half()
+    kc[S // 3] *= 12                                      # a late large key: the running maximum has to move
+    vc = torch.randn(S, 512, device="cuda", generator=g).half()
+    k8 = torch.empty(S, 512, dtype=torch.int8, device="cuda")
+    ksc = torch.empty(8, ks, device="cuda")
+    lk.pf_k8(kc, 0, S, None, ks, k8, ksc)
+    q8 = torch.empty(full, 2048, dtype=torch.int8, device="cuda")
+    qsc, qcs = torch.empty(full, 32, device="cuda"), torch.empty(full, 32, device="cuda")
+    lk.pf_q8(qh, full, None, q8, qsc, qcs)
+
+    def run(rows, given):
+        o = torch.full((full, 2048), 7.0, device="cuda")
+        aqs = torch.full((full, 2048), 7, dtype=torch.int8, device="cuda")
+        asc = torch.full((full, 64, 2), 7.0, device="cuda")
+        note(f"short last block m={rows} P={P} near={near} sink={sink} int8={int8} q8 given={given}")
+        if int8:
+            q = (q8, qsc, qcs) if given else (None, None, None)
+            lk.pf_attn8_q81(*q, qh, rows, P, k8, ksc, ks, kc, vc, near, sink, o, aqs, asc)
+        else:
+            lk.pf_attn_q81(qh, rows, P, kc, vc, o, aqs, asc)
+        torch.cuda.synchronize()
+        return o, aqs, asc
+
+    lk.pf_split_override(-1)
+    lk.pf_pair_override(-1)
+    try:
+        for given in (False, True) if int8 else (False,):
+            for a, b in zip(run(m, given), run(full, given)):
+                assert torch.equal(a[:m].view(torch.uint8), b[:m].view(torch.uint8))
+                assert bool((a[m:] == 7).all())           # nothing past the chunk's rows is written
+    finally:
+        lk.pf_split_override(0)
+        lk.pf_pair_override(0)
