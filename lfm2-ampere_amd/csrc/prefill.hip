@@ -1550,7 +1550,8 @@ static int pf_slots_per_device() {
 // the launch and its merge.  Cutting by T left a remainder per block that
 // started a second round of workgroups (77 rows at 30011, 74 items on 64
 // slots) or, at the cap of 64 pieces, a last piece of all the rest (5 rows at
-// 30000: 90 of 470 tiles).  Attention and merge, by T / by equal pieces, us:
+// 30000: 90 of 470 tiles).  Attention and merge, by T / by equal pieces, us
+// (every block in whole tiles; SHORT has taken up to 10 more off since):
 // 5 rows at 30000 206 / 36.6, 77 at 30011 64.5 (eight-group merge) / 51.5, 300
 // at 9000 60.0 / 48.8, 16 at 3000 21.8 / 17.8, 400 at 0 20.5 / 17.8, 700 at
 // 700 34.1 / 31.3; but 600 at 0 21.7 / 22.4, 1000 at 0 27.3 / 29.0, 900 at
@@ -1590,7 +1591,8 @@ static void pf_plan(int m, int P, int near, int sink, bool int8, bool q81, int s
     };
     // pieces per block (64 left the last piece of a single block of 400 tiles
     // and more up to 130 of them: the attention and merge of a Q8_1 launch of 5
-    // rows at 30000 209 -> 47.8 us, 40 at 26000 174 -> 40.2, 20 at 60000 240 -> 69.2)
+    // rows at 30000 209 -> 47.8 us, 40 at 26000 174 -> 40.2, 20 at 60000 240 -> 69.2,
+    // and 32.9 and 50.8 for 5 and 20 rows with SHORT)
     constexpr int MAXP = 96;
     int cut[PF_MAX_QB][MAXP + 1];                      // piece boundaries per block
     int npc[PF_MAX_QB];
