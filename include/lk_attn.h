@@ -359,8 +359,8 @@ int lk_pf_ctx_buffers(const lk_pf_ctx * ctx, int layer, void ** qh, int8_t ** k8
 int lk_pf_qk_i32(const int8_t * q8, int m, const int8_t * k8, int n,
                  int32_t * s, void * stream);
 
-/* The split work list lk_pf_attn8 (int8 != 0) or lk_pf_attn (fp32 rows; a launch
- * that emits Q8_1 may cut otherwise) would launch for a chunk (m, P, near, sink), under the current lk_pf_split_override and for
+/* The split work list lk_pf_attn8 (int8 != 0) or lk_pf_attn would launch for
+ * a chunk (m, P, near, sink), under the current lk_pf_split_override and for
  * the current device's slot count (512 when no device is visible): items in
  * dispatch order as int32 quadruples (query block, first key tile, end key
  * tile, partial slot or -1) into items[4 * max_items].  Returns the item count

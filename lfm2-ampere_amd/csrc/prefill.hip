@@ -1537,34 +1537,23 @@ static int pf_slots_per_device() {
 //
 // Automatic plan.  Cost model, in units of one int8 tile on a CU shared by
 // two workgroups (from per-workgroup timestamps on MI355X): int8 tile 1,
-// exact or mixed tile 1.4, start-up of a workgroup 2.1.  A kv head has
-// slots/8 workgroup slots (a slot: one of the two workgroups of a CU).
-// Many blocks: T = total cost / slots; when the costliest block
-// exceeds 1.25 T (a causal chunk with P small against m), every block costlier
-// than T is cut into pieces of cost T, from its first tile on, and the rest;
-// items are dispatched costliest first, so the remainders and the short blocks
-// fill the slots that free up early.  (A dispatch simulation calibrated on the
-// measured spans of the C4 chunk: 113 -> 100 us, the floor being ~89.)
-// Few blocks (up to 8, up to 12 where the chunk is no triangle) and fp32 rows
-// as the only output: pieces of equal cost, of the size in a short list that minimises the modelled time of
-// the launch and its merge.  Cutting by T left a remainder per block that
-// started a second round of workgroups (77 rows at 30011, 74 items on 64
-// slots) or, at the cap of 64 pieces, a last piece of all the rest (5 rows at
-// 30000: 90 of 470 tiles).  Attention and merge, by T / by equal pieces, us
-// (every block in whole tiles; SHORT has taken up to 10 more off since):
-// 5 rows at 30000 206 / 36.6, 77 at 30011 64.5 (eight-group merge) / 51.5, 300
-// at 9000 60.0 / 48.8, 16 at 3000 21.8 / 17.8, 400 at 0 20.5 / 17.8, 700 at
-// 700 34.1 / 31.3; but 600 at 0 21.7 / 22.4, 1000 at 0 27.3 / 29.0, 900 at
-// 20000 (fp16) 196 / 202, where T keeps the slots filled.  Launches that emit
-// Q8_1 keep the cuts by T: a row's fp16 probabilities round differently under
-// other cuts (1.3% of the quants of a 30000-key row move by one), and stored
-// Q8_1 planes stay reproducible.
-// Pieces grow when the parts would not fit the partial buffer or the item list.
+// exact or mixed tile 1.4, start-up of a workgroup 2.1.  T = total cost / the
+// slots one kv head gets (a slot: one of the two workgroups of a CU).  When
+// the costliest block exceeds 1.25 T (a causal chunk with P small against
+// m), every block costlier than T is cut into pieces of cost T, from its
+// first tile on, and the rest; items are dispatched costliest first, so the
+// remainders and the short blocks fill the slots that free up early.  (A
+// dispatch simulation calibrated on the measured spans of the C4 chunk: 113 ->
+// 100 us, the floor being ~89.)  T grows when the parts would not fit the
+// partial buffer or the item list.
+// The cuts depend on the chunk and the score type alone, not on which outputs
+// are asked for: p is rounded to fp16 against the running offset of its piece,
+// so under other cuts a row moves by that rounding (rel 1e-4 to 3e-4; 1.3% of
+// the quants of a 30000-key row by one).
 #ifndef PF_PLAN_T
 #define PF_PLAN_T 1.0f      // piece cost, in units of the mean cost per slot
 #endif
-#define PF_FEW 12
-static void pf_plan(int m, int P, int near, int sink, bool int8, bool q81, int split_override, size_t cap_floats,
+static void pf_plan(int m, int P, int near, int sink, bool int8, int split_override, size_t cap_floats,
                     PfWork & wk) {
     wk.n_items = 0; wk.n_split = 0;
     const int nq = (m + PF_BQ - 1) / PF_BQ;
@@ -1573,27 +1562,19 @@ static void pf_plan(int m, int P, int near, int sink, bool int8, bool q81, int s
         return (!int8 || lk_pf_exact(P, 2 * qt, kt, near, sink)) ? 1.4f : 1.0f;
     };
     constexpr float START = 2.1f;
-    // first tile of the run of exact tiles that ends a block (lk_pf_exact)
-    auto kexact = [&](int qt) -> int {
-        if (!int8) return 0;
-        const int lim = P + 2 * qt * 32 - near;               // exact iff kt*64 + 64 > lim
-        return (lim < 64) ? 0 : (lim - 64) / 64 + 1;
-    };
     // cost of key tiles [a, b) of block qt in closed form: the exact tiles of a
     // block are tile 0 with the sink and the run from the first tile within
-    // `near` of the block's first 32 queries to the end
+    // `near` of the block's first 32 queries to the end (lk_pf_exact)
     auto rcost = [&](int qt, int a, int b) -> float {
-        const int kex = kexact(qt);
+        if (!int8) return START + 1.4f * (float) (b - a);
+        const int lim = P + 2 * qt * 32 - near;               // exact iff kt*64 + 64 > lim
+        const int kex = (lim < 64) ? 0 : (lim - 64) / 64 + 1;  // first such tile
         int nex = b - ((a > kex) ? a : kex);
         nex = (nex > 0) ? nex : 0;
-        if (int8 && sink && a == 0 && kex > 0 && b > 0) ++nex;   // tile 0, outside the run
+        if (sink && a == 0 && kex > 0 && b > 0) ++nex;           // tile 0, outside the run
         return START + (float) (b - a) + 0.4f * (float) nex;
     };
-    // pieces per block (64 left the last piece of a single block of 400 tiles
-    // and more up to 130 of them: the attention and merge of a Q8_1 launch of 5
-    // rows at 30000 209 -> 47.8 us, 40 at 26000 174 -> 40.2, 20 at 60000 240 -> 69.2,
-    // and 32.9 and 50.8 for 5 and 20 rows with SHORT)
-    constexpr int MAXP = 96;
+    constexpr int MAXP = 64;                           // pieces per block
     int cut[PF_MAX_QB][MAXP + 1];                      // piece boundaries per block
     int npc[PF_MAX_QB];
     auto fits = [&]() {
@@ -1613,70 +1594,6 @@ static void pf_plan(int m, int P, int near, int sink, bool int8, bool q81, int s
                 for (int p = 0; p <= np; ++p) cut[qt][p] = (p * per < nkt) ? p * per : nkt;
             }
             if (ok && fits()) break;
-        }
-    } else if (!q81 && (nq <= 8 || (nq <= PF_FEW && P >= m))) {
-        const int slots = pf_slots_per_device() / LK_N_KV_HEADS;
-        // of each block: tile cost in units, us per part of the merge (a part's
-        // 8 x 67.6 KB, as many rows as the block has, written and read back),
-        // key tiles
-        float bc[PF_FEW], tpart[PF_FEW], work = 0.0f, cmax = 0.0f;
-        int nk[PF_FEW];
-        for (int qt = 0; qt < nq; ++qt) {
-            nk[qt] = pf_nkt(qt, m, P);
-            bc[qt] = rcost(qt, 0, nk[qt]) - START;
-            tpart[qt] = 0.25f / PF_BQ * (float) std::min(PF_BQ, m - qt * PF_BQ);
-            work += bc[qt];
-            cmax = (bc[qt] > cmax) ? bc[qt] : cmax;
-        }
-        // pieces of block qt when no piece is to cost more than w
-        auto pieces = [&](int qt, float w) -> int {
-            int np = (int) (bc[qt] / w);
-            if ((float) np * w < bc[qt]) ++np;
-            np = np < 1 ? 1 : np > MAXP ? MAXP : np;
-            return np < nk[qt] ? np : nk[qt];
-        };
-        // Modelled us of the launch and its merge (4 us and the parts' traffic):
-        // up to one workgroup per CU, the longest piece at 1.0 us a tile on an
-        // idle chip to 1.75 on a full one; else 2.0 us a unit, of the largest
-        // piece in one round of the slots, of the mean load and half a piece
-        // in more.
-        float best = 0.0f, wbest = 0.0f;
-        auto consider = [&](float w) {
-            int items = 0, parts = 0;
-            float pmax = 0.0f, kmax = 0.0f, merge = 0.0f;
-            for (int qt = 0; qt < nq; ++qt) {
-                const int np = pieces(qt, w);
-                items += np;
-                if (np > 1) { parts += np; merge += tpart[qt] * (float) np; }
-                pmax = std::max(pmax, bc[qt] / (float) np);
-                kmax = std::max(kmax, (float) nk[qt] / (float) np);
-            }
-            if (items > PF_MAX_ITEMS || (size_t) parts * LK_N_KV_HEADS * PF_PART_SLOT > cap_floats) return;
-            float span = START + pmax;
-            if (items > slots)
-                span = std::max(span, (work + START * (float) items) / (float) slots + 0.5f * span);
-            const float fill = 2.0f * (float) items / (float) slots;
-            const float t = (fill > 1.0f ? 2.0f * span : 2.8f + (1.0f + 0.75f * fill) * kmax) + (parts ? 4.0f + merge : 0.0f);
-            if (wbest == 0.0f || t < best) { best = t; wbest = w; }
-        };
-        consider(cmax);                                // unsplit
-        // whole numbers of pieces of the costliest block, growing by about 12%
-        for (int np = 2; np <= MAXP; np += 1 + np / 8) consider(cmax / (float) np * 1.0001f);
-        for (int qt = 0; qt < nq; ++qt) {
-            const int nkt = nk[qt], kdiag = (P + qt * PF_BQ) / PF_BK, kex = kexact(qt);
-            int np = pieces(qt, wbest), n = 0;
-            const float lead = (int8 && sink && kex > 0) ? 0.4f : 0.0f;   // tile 0's extra cost
-            cut[qt][0] = 0;
-            for (int p = 1; p < np; ++p) {
-                // the tile nearest to cost share p/np: int8 tiles up to kex, exact ones after
-                const float c = bc[qt] * (float) p / (float) np - lead;
-                const float kt = c <= (float) kex ? c : (float) kex + (c - (float) kex) / 1.4f;
-                int b = (int) (kt + 0.5f);
-                b = b > kdiag ? kdiag : b;             // no piece starts past the first diagonal tile
-                if (b > cut[qt][n] && b < nkt) cut[qt][++n] = b;
-            }
-            cut[qt][++n] = nkt;
-            npc[qt] = n;
         }
     } else {
         float total = 0.0f, cmax = 0.0f;
@@ -1736,7 +1653,7 @@ static void pf_plan(int m, int P, int near, int sink, bool int8, bool q81, int s
 extern "C" int lk_pf_plan_items(int m, int P, int near, int sink, int int8, int32_t * items, int max_items) {
     if (m < 1 || P < 0 || max_items < 0 || (!items && max_items > 0)) return -1;
     PfWork wk;
-    pf_plan(m, P, near, sink, int8 != 0, false, g_pf_split_override.load(std::memory_order_relaxed), PF_PART_CAP, wk);
+    pf_plan(m, P, near, sink, int8 != 0, g_pf_split_override.load(std::memory_order_relaxed), PF_PART_CAP, wk);
     for (int i = 0; i < wk.n_items && i < max_items; ++i) {
         items[4 * i + 0] = (int32_t) (wk.item[i] & 255);
         items[4 * i + 1] = (int32_t) (wk.krange[i] & 0xffff);
@@ -1790,7 +1707,7 @@ static int pf_attn_launch(const int8_t * q8, const float * qsc, const float * qc
     // a caller workspace bounds the partials the plan may write (a smaller one
     // gives coarser pieces, none at all an unsplit launch); without one the
     // library's static scratch is used
-    pf_plan(m, P, near, sink, INT8, Q81, split_override, work ? work_bytes / sizeof(float) : (size_t) PF_PART_CAP, wk);
+    pf_plan(m, P, near, sink, INT8, split_override, work ? work_bytes / sizeof(float) : (size_t) PF_PART_CAP, wk);
     const int nq = (m + PF_BQ - 1) / PF_BQ, last = m - (nq - 1) * PF_BQ;
     // at most 32 rows in the last block: the kernel that skips its empty query
     // blocks (from 33 rows on there is nothing it could skip)

@@ -132,3 +132,35 @@ def test_short_last_block_is_bit_identical(lk, m, P, near, sink, int8):
     finally:
         lk.pf_split_override(0)
         lk.pf_pair_override(0)
+
+
+# Asking for the Q8_1 planes changes no row: the key-range cuts are those of the
+# chunk, for both score types, on chunks of few blocks whose plan splits.
+@pytest.mark.parametrize("m,P", [(5, 30000), (77, 3000), (77, 30011), (300, 9000), (700, 700)])
+@pytest.mark.parametrize("int8", [True, False])
+def test_rows_do_not_depend_on_the_planes(lk, m, P, int8):
+    S, ks = P + m, lk.kstride_for(P + m)
+    g = torch.Generator(device="cuda").manual_seed(m + P)
+    qh = (torch.randn(m, 2048, device="cuda", generator=g) / 4).half()
+    kc = torch.randn(S, 512, device="cuda", generator=g).half()
+    vc = torch.randn(S, 512, device="cuda", generator=g).half()
+    assert lk.pf_plan_items(m, P, 1024, 1, int8)
+    o1, o2 = (torch.full((m, 2048), float("nan"), device="cuda") for _ in range(2))
+    aqs = torch.empty(m, 2048, dtype=torch.int8, device="cuda")
+    asc = torch.empty(m, 64, 2, device="cuda")
+    note(f"rows with and without planes m={m} P={P} int8={int8}")
+    if int8:
+        k8 = torch.empty(S, 512, dtype=torch.int8, device="cuda")
+        ksc = torch.empty(8, ks, device="cuda")
+        lk.pf_k8(kc, 0, S, None, ks, k8, ksc)
+        lk.pf_attn8(None, None, None, qh, m, P, k8, ksc, ks, kc, vc, 1024, 1, o1)
+        lk.pf_attn8_q81(None, None, None, qh, m, P, k8, ksc, ks, kc, vc, 1024, 1, o2, aqs, asc)
+    else:
+        lk.pf_attn(qh, m, P, kc, vc, o1)
+        lk.pf_attn_q81(qh, m, P, kc, vc, o2, aqs, asc)
+    torch.cuda.synchronize()
+    assert torch.equal(o1.view(torch.int32), o2.view(torch.int32))
+    qs, sc = torch.empty_like(aqs), torch.empty_like(asc)
+    lk.pf_quant_rows(o1, m, 2048, 64, qs, sc)
+    torch.cuda.synchronize()
+    assert torch.equal(qs, aqs) and torch.equal(sc.view(torch.int32), asc.view(torch.int32))
