@@ -295,23 +295,25 @@ __device__ __forceinline__ uint32_t lk_lds_addr(const void * p) {
 // lds + 16*lane (lds must be wave-uniform).  Issued as inline asm so the
 // compiler does not serialise later LDS reads on it; completion is tracked by
 // hand with vmcnt (in-order) plus a barrier.  M0 is written here; no other
-// code in this library uses M0, so clobbering it is safe.  lk_dma16 is
+// code in this library uses M0, so clobbering it is safe.  An LDS DMA needs one
+// wait state after the scalar write of M0 (the s_nop): the compiler inserts it
+// for its own DMAs but does not look inside asm.  lk_dma16 is
 // non-temporal (streams read once), lk_dma16c keeps the normal cache policy
 // (tiles that other workgroups read again).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void lk_dma16(const void * src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
                  :: "v"(src), "s"(lds) : "memory", "m0");
 }
 __device__ __forceinline__ void lk_dma16c(const void * src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :: "v"(src), "s"(lds) : "memory", "m0");
 }
 // The same with a wave-uniform 64-bit base (SGPRs) plus a per-lane 32-bit
 // byte offset: moving the source costs only scalar adds.
 __device__ __forceinline__ void lk_dma16c_so(const void * sbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop

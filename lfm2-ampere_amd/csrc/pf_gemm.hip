@@ -83,7 +83,7 @@ __device__ __forceinline__ constexpr int pfg_slot(int n, int row, int x) { retur
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void pfg_dma4(const void * sbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop

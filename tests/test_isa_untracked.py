@@ -129,3 +129,23 @@ def test_untracked_loads_with_the_makefiles_own_flags(tmp_path):
         loads, first_wait = _check_paths(name, body)
         assert loads == (20 if fused else 4), (name, loads)
         assert first_wait == 12, (name, first_wait)
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+@pytest.mark.parametrize("src,floor", [("decode", 16), ("prefill", 100), ("pf_gemm", 40)])
+def test_a_wait_state_between_m0_and_the_lds_dma(tmp_path, src, floor):
+    """An LDS DMA takes its LDS address from M0 and needs one wait state after the
+    scalar write of M0.  The compiler keeps it for its own DMAs but does not look
+    inside inline asm, which therefore has to hold the wait state itself."""
+    cmd = next(l for l in subprocess.run(["make", "-n", "-B", "_build/%s.hip.o" % src], cwd=PKG, check=True,
+                                         capture_output=True, text=True).stdout.split("\n") if " -c -x hip " in l)
+    args = cmd.split(" 2>&1")[0].replace("-c -x hip", "--offload-device-only -S -x hip").split()
+    asm = tmp_path / (src + ".s")
+    args[args.index("-o") + 1] = str(asm)
+    subprocess.run(args, check=True, cwd=PKG, capture_output=True)
+    ins = [t for t in (l.split(";")[0].strip() for l in asm.read_text().split("\n"))
+           if t and not t.startswith(".") and not t.endswith(":")]
+    dma = [k for k, t in enumerate(ins) if re.match(r"(global|buffer)_load_lds|buffer_load.* lds\b", t)]
+    assert len(dma) >= floor
+    for k in dma:
+        assert not re.match(r"s_\w+ m0,", ins[k - 1]), ins[k - 1:k + 1]
