@@ -1156,111 +1156,127 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
     }
 }
 
-// Merge of the parts of split query blocks: a thread holds (head, row) over 32
-// dims -- one Q8_1 block; the parts are weighted 2^(m_p - M) with the exact max
-// M and summed in a fixed order.  Bound by memory latency: a thread's loads of
-// up to MAXP parts are independent, one round trip per pass.
-//   NPG 1: workgroup (split block, kv head, half of the dims), threads (head,
-//          row), four parts per pass.
-//   NPG 8: one workgroup per head as well, threads (part group, row): group g
-//          sums parts g, g + 8, ..., two per pass, and the 8 sums are merged
-//          through LDS in group order.  For launches of more than 8 parts per
-//          block, a short chunk deep in a prompt: 77 rows at position 30011
-//          (37 parts) 29.6 -> 11.2 us, 5 rows at 30000 (64 parts) 52.3 -> 10.7,
-//          300 at 9000 (15) 12.9 -> 10.4; with 4 to 5 parts its LDS pass
-//          loses (1100 rows at 3333 11.7 -> 16.5, 1500 at 0 10.6 -> 16.1).
-#define PF_CMB_LD 36                                      // floats per (group, row) in LDS: 32 dims, m, l, pad
-template <int NPG>
-__global__ void __launch_bounds__(NPG == 1 ? 256 : 64 * NPG)
+// Merge of the parts of split query blocks, in passes of four parts: the running
+// maximum M takes in the pass's maxima, L and the sums are rescaled by 2^(old M
+// - M), then the pass's parts are added in part order, weighted 2^(m_p - M).
+// Both forms do exactly this for every value, so they give the same bits.
+// Bound by memory latency; what a form chooses is how many loads of a thread
+// are in flight.
+//   narrow: workgroup (split block, kv head, half of the dims), threads (head,
+//           row) over 32 dims, one Q8_1 block; four parts per round trip.
+//   WIDE:   one workgroup per head as well, threads (4 of the 32 dims, row): the
+//           next eight parts load while eight are added, and the Q8_1 block is
+//           gathered through LDS.  For launches of more than 8 parts per block,
+//           a short chunk deep in a prompt.  Narrow / wide, us: 5 rows at 30000
+//           (64 parts) 55.8 / 12.9, 77 at 30011 (34) 26.8 / 9.2, 141 at 25060
+//           (22) 18.0 / 8.0, 300 at 9000 (15) 13.5 / 11.0, 77 at 3000 (10) 10.3
+//           / 5.7; with 5 parts a block the second eight are idle: 1100 at 3333
+//           13.3 / 14.2, 1500 at 0 12.2 / 14.0.  Sixteen at a time without the
+//           overlap: 18.1 at 64 parts, 12.8 at 15.
+#define PF_CMB_LD 36                                      // floats per row in LDS: 32 dims and a pad
+template <bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 512 : 256)
 lk_k_pf_combine(const float * __restrict__ pbuf, int m, int P, const PfWork work, float * __restrict__ o,
                 int8_t * __restrict__ aqs, float2 * __restrict__ asc) {
 #pragma clang fp contract(off)
+    constexpr int NC = WIDE ? 1 : 8;                      // 4-dim chunks per thread
+    constexpr int NP = WIDE ? 8 : 4;                      // parts loaded at once
     const int kvh = blockIdx.y, hb = blockIdx.z & 1;      // dims 32hb .. 32hb+31
     const int qt = work.split_qt[blockIdx.x];
     const int slot = work.slot0[qt];
-    const int row = threadIdx.x & 63, h = NPG == 1 ? threadIdx.x >> 6 : blockIdx.z >> 1;
-    const int pg = NPG == 1 ? 0 : threadIdx.x >> 6;
+    const int row = threadIdx.x & 63, h = WIDE ? blockIdx.z >> 1 : threadIdx.x >> 6;
+    const int c0 = WIDE ? threadIdx.x >> 6 : 0;
     const int qr = qt * PF_BQ + row;
-    if (NPG == 1 && qr >= m) return;
+    if (!WIDE && qr >= m) return;
     const int np = qr < m ? work.nparts[qt] : 0;          // rows past m hold nothing
     auto base = [&](int p) { return pbuf + (size_t) ((slot + p) * LK_N_KV_HEADS + kvh) * PF_PART_SLOT; };
     float M = -INFINITY, L = 0.0f;
-    lk_f4 A[8] = {};
-    // one pass over parts p0, p0 + NPG, ... (W of them): all loads first (one
-    // memory round trip), then the merge in part order
-    auto pass = [&](auto wc, int p0) {
+    lk_f4 A[NC] = {};
+    // parts [p0, p0 + W): the loads, one memory round trip ...
+    auto load = [&](auto wc, int p0, auto & ml, auto & a) {
         constexpr int W = decltype(wc)::value;
-        float2 ml[W];
-        lk_f4 a[W][8];
 #pragma unroll
         for (int i = 0; i < W; ++i) {
-            const int p = (p0 + i * NPG < np) ? p0 + i * NPG : p0;   // clamped: loads stay in bounds
+            const int p = (p0 + i < np) ? p0 + i : p0;    // clamped: loads stay in bounds
             ml[i] = ((const float2 *) (base(p) + PF_PART_ACC))[h * PF_BQ + row];
-            const lk_f4 * src = (const lk_f4 *) base(p) + (size_t) (h * 16 + 8 * hb) * PF_BQ + row;
+            const lk_f4 * src = (const lk_f4 *) base(p) + (size_t) (h * 16 + 8 * hb + c0) * PF_BQ + row;
 #pragma unroll
-            for (int c = 0; c < 8; ++c) a[i][c] = src[c * PF_BQ];
+            for (int c = 0; c < NC; ++c) a[i][c] = src[c * PF_BQ];
         }
-        float Mn = M;
-#pragma unroll
-        for (int i = 0; i < W; ++i) if (p0 + i * NPG < np) Mn = fmaxf(Mn, ml[i].x);
-        const float r = lk_exp2(M - Mn);                  // 0 on the first pass (M = -inf)
-        L *= r;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) A[c] *= r;
-#pragma unroll
-        for (int i = 0; i < W; ++i) {
-            if (p0 + i * NPG >= np) break;
-            const float wgt = lk_exp2(ml[i].x - Mn);
-            L += ml[i].y * wgt;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) A[c] += a[i][c] * wgt;
-        }
-        M = Mn;
     };
-    if constexpr (NPG == 1) {
-        // two parts per block is the common case: no redundant loads for it
-        if (np == 2) pass(std::integral_constant<int, 2>{}, 0);
-        else for (int p0 = 0; p0 < np; p0 += 4) pass(std::integral_constant<int, 4>{}, p0);
-    } else {
-        for (int p0 = pg; p0 < np; p0 += 2 * NPG) pass(std::integral_constant<int, 2>{}, p0);
-        // (a group without parts holds M = -inf, L = 0, A = 0: weight 0 below)
-        __shared__ __attribute__((aligned(16))) float s_g[NPG][PF_BQ][PF_CMB_LD];
-        float * G = s_g[pg][row];
+    // ... and their merge, up to four parts a pass
+    auto add = [&](auto wc, int p0, const auto & ml, const auto & a) {
+        constexpr int W = decltype(wc)::value, PASS = W < 4 ? W : 4;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) *(lk_f4 *) (G + 4 * c) = A[c];
-        *(float2 *) (G + 32) = make_float2(M, L);
-        __syncthreads();
-        if (pg != 0 || qr >= m) return;
+        for (int k = 0; k < W; k += PASS) {
+            if (p0 + k >= np) break;
+            float Mn = M;
 #pragma unroll
-        for (int g = 1; g < NPG; ++g) M = fmaxf(M, s_g[g][row][32]);
-        L = 0.0f;
+            for (int i = k; i < k + PASS; ++i) if (p0 + i < np) Mn = fmaxf(Mn, ml[i].x);
+            const float r = lk_exp2(M - Mn);              // 0 on the first pass (M = -inf)
+            L *= r;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) A[c] = (lk_f4){ 0.f, 0.f, 0.f, 0.f };
+            for (int c = 0; c < NC; ++c) A[c] *= r;
 #pragma unroll
-        for (int g = 0; g < NPG; ++g) {
-            const float * E = s_g[g][row];
-            const float2 ml = *(const float2 *) (E + 32);
-            const float wgt = lk_exp2(ml.x - M);
-            L += ml.y * wgt;
+            for (int i = k; i < k + PASS; ++i) {
+                if (p0 + i >= np) break;
+                const float wgt = lk_exp2(ml[i].x - Mn);
+                L += ml[i].y * wgt;
 #pragma unroll
-            for (int c = 0; c < 8; ++c) A[c] += *(const lk_f4 *) (E + 4 * c) * wgt;
+                for (int c = 0; c < NC; ++c) A[c] += a[i][c] * wgt;
+            }
+            M = Mn;
         }
+    };
+    using N = std::integral_constant<int, NP>;
+    if constexpr (WIDE) {
+        if (np > 0) {
+            float2 ml[2][NP];
+            lk_f4 a[2][NP][NC];
+            load(N{}, 0, ml[0], a[0]);
+            for (int p0 = 0; p0 < np; p0 += 2 * NP) {
+                if (p0 + NP < np) load(N{}, p0 + NP, ml[1], a[1]);
+                add(N{}, p0, ml[0], a[0]);
+                if (p0 + NP >= np) break;
+                if (p0 + 2 * NP < np) load(N{}, p0 + 2 * NP, ml[0], a[0]);
+                add(N{}, p0 + NP, ml[1], a[1]);
+            }
+        }
+    } else {
+        auto parts = [&](auto wc, int p0) {
+            float2 ml[decltype(wc)::value];
+            lk_f4 a[decltype(wc)::value][NC];
+            load(wc, p0, ml, a);
+            add(wc, p0, ml, a);
+        };
+        // two parts per block is the common case: no redundant loads for it
+        if (np == 2) parts(std::integral_constant<int, 2>{}, 0);
+        else for (int p0 = 0; p0 < np; p0 += NP) parts(N{}, p0);
     }
     const float il = 1.0f / L;
-    float x[32];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const lk_f4 v = A[c] * il;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x[4 * c + r] = v[r];
-    }
     const size_t col0 = (size_t) (kvh * LK_G + h) * LK_HEAD_DIM + 32 * hb;
-    if (o) {
-        float * dst = o + (size_t) qr * LK_HIDDEN + col0;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) *(float4 *) (dst + 4 * c) = make_float4(x[4 * c], x[4 * c + 1], x[4 * c + 2], x[4 * c + 3]);
+    for (int c = 0; c < NC; ++c) A[c] = A[c] * il;
+    if (o && qr < m) {
+        float * dst = o + (size_t) qr * LK_HIDDEN + col0 + 4 * c0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) *(lk_f4 *) (dst + 4 * c) = A[c];
     }
     if (aqs) {                                            // the block's Q8_1, in-thread, same tree
+        float x[32];
+        if constexpr (WIDE) {
+            __shared__ __attribute__((aligned(16))) float s_x[PF_BQ][PF_CMB_LD];
+            *(lk_f4 *) (s_x[row] + 4 * c0) = A[0];
+            __syncthreads();
+            if (c0 != 0 || qr >= m) return;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) *(lk_f4 *) (x + 4 * c) = *(const lk_f4 *) (s_x[row] + 4 * c);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[4 * c + r] = A[c][r];
+        }
         float am = 0.0f;
 #pragma unroll
         for (int i = 0; i < 32; ++i) am = fmaxf(am, fabsf(x[i]));
@@ -1732,10 +1748,10 @@ static int pf_attn_launch(const int8_t * q8, const float * qsc, const float * qc
     int npmax = 0;
     for (int i = 0; i < wk.n_split; ++i) npmax = std::max(npmax, (int) wk.nparts[wk.split_qt[i]]);
     if (npmax <= 8)
-        hipLaunchKernelGGL(lk_k_pf_combine<1>, dim3(wk.n_split, LK_N_KV_HEADS, 2), dim3(256), 0, st,
+        hipLaunchKernelGGL(lk_k_pf_combine<false>, dim3(wk.n_split, LK_N_KV_HEADS, 2), dim3(256), 0, st,
                            (const float *) pbuf, m, P, wk, o, aqs, asc);
     else
-        hipLaunchKernelGGL(lk_k_pf_combine<8>, dim3(wk.n_split, LK_N_KV_HEADS, 2 * LK_G), dim3(512), 0, st,
+        hipLaunchKernelGGL(lk_k_pf_combine<true>, dim3(wk.n_split, LK_N_KV_HEADS, 2 * LK_G), dim3(512), 0, st,
                            (const float *) pbuf, m, P, wk, o, aqs, asc);
     rc = lk_launch_status(what);
     if (rc) return rc;

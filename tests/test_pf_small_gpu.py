@@ -51,10 +51,10 @@ def test_quant_rows_bit_exact(lk, oracle, rows, kb, pad, offset):
     assert np.array_equal(host(sc).view(np.uint32), np.asarray(ws, np.float32).reshape(rows, kb, 2).view(np.uint32))
 
 
-# more than 8 parts per block take the part-group merge: part counts off its 8
-# groups of two, ragged last blocks, both outputs.  2e-3 of the largest output
-# is the bound every prefill case here is held to: p rounded to fp16 (2^-11
-# each) on rows of a few thousand keys.
+# more than 8 parts per block take the wide merge: part counts off its two
+# eights, ragged last blocks, both outputs.  2e-3 of the largest output is the
+# bound every prefill case here is held to: p rounded to fp16 (2^-11 each) on
+# rows of a few thousand keys.
 @pytest.mark.parametrize("m,P,tiles", [(1, 640, 1), (5, 2100, 2), (77, 1500, 1), (130, 3000, 3), (64, 4000, 1)])
 def test_combine_many_parts(lk, oracle, m, P, tiles):
     from gpu_util import dev_h
@@ -164,3 +164,54 @@ def test_rows_do_not_depend_on_the_planes(lk, m, P, int8):
     lk.pf_quant_rows(o1, m, 2048, 64, qs, sc)
     torch.cuda.synchronize()
     assert torch.equal(qs, aqs) and torch.equal(sc.view(torch.int32), asc.view(torch.int32))
+
+
+# The merge adds the parts in part order, four a pass, whatever their number: the
+# same recurrence on the partials that the launch left in the caller's workspace
+# gives the same bits.  One tile per part; part counts on both sides of the wide
+# merge's line and of its eights.
+@pytest.mark.parametrize("m,P,parts", [(5, 120, [2]), (64, 128, [3]), (5, 500, [8]), (5, 570, [9]), (5, 1010, [16]),
+                                       (20, 1060, [17]), (77, 2112, [34, 35]), (40, 2960, [47]), (1, 4095, [64])])
+def test_merge_is_the_part_order_recurrence(lk, m, P, parts):
+    S = P + m
+    g = torch.Generator(device="cuda").manual_seed(m + P)
+    qh = (torch.randn(m, 2048, device="cuda", generator=g) / 2).half()
+    kc = torch.randn(S, 512, device="cuda", generator=g).half()
+    vc = torch.randn(S, 512, device="cuda", generator=g).half()
+    o = torch.full((m, 2048), float("nan"), device="cuda")
+    aqs = torch.empty(m, 2048, dtype=torch.int8, device="cuda")
+    asc = torch.empty(m, 64, 2, device="cuda")
+    work = torch.zeros(lk.pf_part_bytes() // 4, device="cuda")
+    note(f"merge order m={m} P={P} parts={parts}")
+    try:
+        lk.pf_split_override(1)
+        items = lk.pf_plan_items(m, P, 0, 0, False)
+        assert [sum(1 for i in items if i[0] == q) for q in range((m + 63) // 64)] == parts
+        lk.pf_attn_ws(qh, m, P, kc, vc, o, aqs, asc, work)
+        torch.cuda.synchronize()
+    finally:
+        lk.pf_split_override(0)
+    ACC, SLOT = 4 * 16 * 64 * 4, 4 * 16 * 64 * 4 + 4 * 64 * 2
+    for qt in {i[0] for i in items}:
+        slots = [i[3] for i in sorted(items) if i[0] == qt]
+        if slots == [-1]:
+            continue
+        rows = min(64, m - 64 * qt)
+        recs = work[slots[0] * 8 * SLOT:(slots[0] + len(slots)) * 8 * SLOT].view(len(slots), 8, SLOT)
+        acc = recs[:, :, :ACC].reshape(-1, 8, 4, 16, 64, 4).permute(0, 1, 2, 4, 3, 5).reshape(-1, 8, 4, 64, 64)
+        ml = recs[:, :, ACC:].reshape(-1, 8, 4, 64, 2)
+        M = torch.full((8, 4, 64), -float("inf"), device="cuda")
+        L, A = torch.zeros_like(M), torch.zeros(8, 4, 64, 64, device="cuda")
+        for p0 in range(0, len(slots), 4):
+            one = range(p0, min(p0 + 4, len(slots)))
+            Mn = M
+            for p in one:
+                Mn = torch.maximum(Mn, ml[p, ..., 0])
+            r = torch.exp2(M - Mn)
+            L, A = L * r, A * r.unsqueeze(-1)
+            for p in one:
+                w = torch.exp2(ml[p, ..., 0] - Mn)
+                L, A = L + ml[p, ..., 1] * w, A + acc[p] * w.unsqueeze(-1)
+            M = Mn
+        want = (A * (1.0 / L).unsqueeze(-1)).permute(2, 0, 1, 3).reshape(64, 2048)[:rows]
+        assert torch.equal(o[64 * qt:64 * qt + rows].view(torch.int32), want.contiguous().view(torch.int32)), len(slots)
