@@ -60,7 +60,9 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     # HIP runtime under the same soname; load it first so the process has one
     # runtime and torch's streams and allocations are valid for the library.
     import torch
-    _raw_stream, _device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+    # (absent from a CPU-only torch, where the host-side entry points still work)
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    _device = getattr(torch._C, "_cuda_getDevice", None)
     lib = ctypes.CDLL(path)
     P, I, S = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t
     sig = {
@@ -138,6 +140,9 @@ def _stream(stream) -> Optional[int]:
     read directly: torch.cuda.current_stream() builds a Stream object, 2.7 us of
     a host path that is otherwise 8 us for a decode call (two launches)."""
     if stream is None:
+        if _raw_stream is None or _device is None:
+            import torch
+            return torch.cuda.current_stream().cuda_stream or None
         return _raw_stream(_device()) or None
     return stream.cuda_stream or None
 

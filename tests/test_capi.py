@@ -4,6 +4,8 @@ CPU only: no kernel is launched here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -163,3 +165,27 @@ def test_python_mirror_fails_loudly_without_library(tmp_path):
             mod.load(str(tmp_path / "missing.so"))
     finally:
         importlib.reload(lk_attn)
+
+
+def test_host_side_works_with_a_torch_without_device_streams():
+    """A CPU-only torch lacks the raw stream handles: the host-side entry points
+    still load and answer, and asking for a stream raises torch's own error."""
+    code = """
+import torch
+for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+    if hasattr(torch._C, name):
+        delattr(torch._C, name)
+import lk_attn as lk
+assert lk.part_bytes() > 0
+def refuse():
+    raise AssertionError("Torch not compiled with CUDA enabled")
+torch.cuda.current_stream = refuse
+try:
+    lk._stream(None)
+except AssertionError as e:
+    print("refused:", e)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT,
+                       env={**os.environ, "PYTHONPATH": os.path.join(ROOT, "lfm2-ampere_amd")})
+    assert r.returncode == 0, r.stderr
+    assert "refused: Torch not compiled" in r.stdout
