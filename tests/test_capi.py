@@ -189,3 +189,21 @@ except AssertionError as e:
                        env={**os.environ, "PYTHONPATH": os.path.join(ROOT, "lfm2-ampere_amd")})
     assert r.returncode == 0, r.stderr
     assert "refused: Torch not compiled" in r.stdout
+
+
+def test_makefile_stamps_one_flag_line_for_every_target(tmp_path):
+    """The stamp of the flag set is the same whichever object is asked for:
+    building one alone leaves the others up to date."""
+    build = str(tmp_path / "b")
+
+    def dry(target):
+        out = subprocess.run(["make", "-n", f"BUILD={build}", f"LIB={tmp_path}/l.so", target], capture_output=True,
+                             text=True, check=True, cwd=os.path.join(ROOT, "lfm2-ampere_amd")).stdout.split("\n")
+        return ([l for l in out if "cmp -s" in l],
+                {re.search(r"csrc/(\w+\.\w+)", l).group(1): "kernarg-preload" in l for l in out if " -c -x hip " in l})
+
+    stamp, flags = dry("all")
+    assert len(stamp) == 1
+    for src, preload in flags.items():
+        assert preload == (src != "prefill.hip")
+        assert dry(f"{build}/{src}.o") == (stamp, {src: preload})
