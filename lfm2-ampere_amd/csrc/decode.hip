@@ -123,10 +123,11 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     // below: vector-memory loads complete in issue order, so a load issued
     // after the DMAs would wait for them (about 3 us at start-up).  This
     // lane's q values (dims 8g+i and 32+8g+i of head 4w + (col & 3)); with the
-    // producer folded in also the rotary frequency of table entry 4w + lane
-    // (lanes 0-3, a scalar load), the q norm weights and, after the slice
-    // plan, the new row's k and v and the k norm weights (used only by the
-    // workgroup whose slice holds the position).
+    // producer folded in also the rotary frequency of table entry 4w +
+    // (lane & 3) (a scalar load), the q norm weights and, after the slice plan,
+    // the new row's k and v and the k norm weights (k is normalised and rotated
+    // in every workgroup beside q; only the one whose slice holds the position
+    // stores it and its v).
     // Loaded untracked (lk_ld16_untracked) and awaited after the DMA issue
     // with a count that leaves the tile DMAs in flight: a tracked load here
     // would make the compiler wait for every tile in flight before the
@@ -161,7 +162,7 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     if constexpr (LK_ATTN_TARGET_N <= LK_DEC_TILE)
         ntile = sp < nt ? (nt - sp + LK_ATTN_SPLIT - 1) / LK_ATTN_SPLIT : 0;
     else
-        ntile = (sp < ns && sp < nt) ? (nt - sp + ns - 1) / ns : 0;
+        ntile = ((nt - sp + ns - 1) / ns) & -(int) ((sp < ns) & (sp < nt));   // masked: a branch has no place here
     // A slice with no tiles (ntile = 0: sp >= nt or sp >= ns) takes the same
     // path with an empty tile loop, so its record is the neutral one (m =
     // -inf, l = 0, acc = 0) and every slot the combine reads is valid without
@@ -170,7 +171,7 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     // be free to reuse their registers (a store address formed in one of
     // them would be overwritten by the arriving data).
     const int pos = seq - 1;
-    const bool own_pos = FUSED && ntile > 0 && sp + ns * (ntile - 1) == nt - 1;   // this slice holds position pos (its last tile)
+    const bool own_pos = FUSED & (ntile > 0) & (sp + ns * (ntile - 1) == nt - 1);   // this slice holds position pos (its last tile)
     if constexpr (FUSED) {          // loaded by every workgroup: see the wait below
         const float * kp = pr.k_src + w * LK_HEAD_DIM + 8 * g;
         const float * vp = pr.v_src + w * LK_HEAD_DIM + 8 * g;
@@ -243,12 +244,13 @@ lk_k_attn_split(const float * __restrict__ q, const _Float16 * kc,
     if constexpr (FUSED) {
         // The 32 (cos, sin) entries of position seq-1, 4 per wave, under the
         // latency of the loads; every lane forms and writes entry 4w +
-        // (lane & 3), so that there is no branch of ours while they are
-        // pending.  With the side-by-side norms below, per layer of the step
-        // graph 10.73 -> 10.04 us at 20 positions, 11.19 -> 10.90 at 2500,
-        // 18.93 -> 18.81 at 32768.
+        // (lane & 3) and lk_sincos has no branch either, so the code stays
+        // straight while they are pending (a test checks the assembly).  With
+        // the side-by-side norms below, per layer of the step graph 10.73 ->
+        // 10.04 us at 20 positions, 11.19 -> 10.90 at 2500, 18.93 -> 18.81 at
+        // 32768.
         float c, sn;
-        lk_rope_angle(pos, rfreq, c, sn);
+        lk_rope_angle_straight(pos, rfreq, c, sn);
         s_c[4 * w + (lane & 3)] = c;
         s_s[4 * w + (lane & 3)] = sn;
     }

@@ -222,9 +222,10 @@ __host__ __device__ __forceinline__ void lk_attn_slices(int seq, int & ns, int &
     0x1.61bea2p-15f, 0x1.ab8884p-16f, 0x1.025b58p-16f, 0x1.383f88p-17f, \
     0x1.796182p-18f, 0x1.c8198cp-19f, 0x1.139e96p-19f, 0x1.4d1c98p-20f, \
     0x1.9298acp-21f, 0x1.e69338p-22f, 0x1.26091cp-22f, 0x1.635e88p-23f
-// Entry i (0..31) by a select tree over the bits of i on immediate constants:
-// no memory access (a load of a constant table went to L2 or HBM at the start
-// of every producer workgroup and cost more than the fp64 pow it replaced).
+// Entry i (0..31) by a select tree over the bits of i.  (The compiler makes the
+// first level 16 independent loads of a constant table, in flight together; one
+// load of a table in constant memory, at the start of every producer workgroup,
+// had cost more than the fp64 pow it replaced.)
 __device__ __forceinline__ float lk_rope_freq(int i) {
     constexpr float T[LK_HEAD_DIM / 2] = { LK_ROPE_FREQ_INIT };
     float v[16];
@@ -246,8 +247,46 @@ __device__ __forceinline__ float lk_rope_freq_quad(int j_uniform, int lane) {
     const float lo = (lane & 1) ? f.y : f.x, hi = (lane & 1) ? f.w : f.z;
     return (lane & 2) ? hi : lo;
 }
-__device__ __forceinline__ void lk_rope_angle(int pos, float f, float & c, float & s) {
+// sin and cos of x in fp64, |x| <= 2^31, without a branch: the decode kernel forms
+// them while untracked loads are pending, and the library's sincos has two
+// (large and small arguments).  Cody and Waite's reduction by the nearest
+// multiple k of pi/2 in two parts -- x is an fp32 number, so x - k*hi is exact
+// (a multiple of 2^-52 below 1) and the second step rounds once -- then the
+// Taylor series, whose first term left out is below 2^-53 of the result on
+// |r| <= pi/4.
+__host__ __device__ __forceinline__ void lk_sincos(double x, double & sn, double & cs) {
+    constexpr double PIO2_HI = 0x1.921fb54442d18p+0, PIO2_LO = 0x1.1a62633145c07p-54;
+    const double k = __builtin_rint(x * 0x1.45f306dc9c883p-1);             // 2/pi
+    const double r = __builtin_fma(-k, PIO2_LO, __builtin_fma(-k, PIO2_HI, x)), z = r * r;
+    constexpr double S[7] = { -1.0 / 1307674368000, 1.0 / 6227020800, -1.0 / 39916800, 1.0 / 362880, -1.0 / 5040,
+                              1.0 / 120, -1.0 / 6 };                       // (-1)^n / (2n+1)!, n = 7 .. 1
+    constexpr double C[8] = { 1.0 / 20922789888000, -1.0 / 87178291200, 1.0 / 479001600, -1.0 / 3628800, 1.0 / 40320,
+                              -1.0 / 720, 1.0 / 24, -1.0 / 2 };            // (-1)^n / (2n)!, n = 8 .. 1
+    double s = S[0], c = C[0];
+#pragma unroll
+    for (int n = 1; n < 7; ++n) s = __builtin_fma(s, z, S[n]);
+#pragma unroll
+    for (int n = 1; n < 8; ++n) c = __builtin_fma(c, z, C[n]);
+    s = __builtin_fma(r * z, s, r);
+    c = __builtin_fma(c, z, 1.0);
+    const int q = (int) k;
+    const double u = (q & 1) ? c : s, v = (q & 1) ? s : c;
+    sn = (q & 2) ? -u : u;
+    cs = ((q + 1) & 2) ? -v : v;
+}
+// The entry by lk_sincos (decode) and by the library's sincos (the table of the
+// stand-alone producers); the fp32 results are the same bits (all positions
+// below 2^24 compared on the device).  In the producers' kernel lk_sincos makes
+// the compiler wait between the loads of lk_rope_freq: 4096 rows 15.8 -> 19.6 us.
+__host__ __device__ __forceinline__ void lk_rope_angle_straight(int pos, float f, float & c, float & s) {
     const float a = (float) pos * f;                           // fp32 product, as the reference
+    double sd, cd;
+    lk_sincos((double) a, sd, cd);
+    c = (float) cd;
+    s = (float) sd;
+}
+__device__ __forceinline__ void lk_rope_angle(int pos, float f, float & c, float & s) {
+    const float a = (float) pos * f;
     double sd, cd;
     sincos((double) a, &sd, &cd);
     c = (float) cd;

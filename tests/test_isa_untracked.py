@@ -149,3 +149,32 @@ def test_a_wait_state_between_m0_and_the_lds_dma(tmp_path, src, floor):
     assert len(dma) >= floor
     for k in dma:
         assert not re.match(r"s_\w+ m0,", ins[k - 1]), ins[k - 1:k + 1]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+@pytest.mark.parametrize("knobs", [[], ["TARGET_N=128"], ["SPLIT=128"], ["NBUF=2"], ["NBUF=3"], ["TILE=32", "NBUF=2"],
+                                   ["TILE=32", "NBUF=2", "TARGET_N=64"]], ids=lambda k: "_".join(k) or "default")
+def test_no_branch_while_untracked_loads_are_pending(tmp_path, knobs):
+    """Between the untracked loads and their wait the code is straight: around a
+    branch the compiler may copy registers that are still in flight.  Checked,
+    with the registers themselves, at the default and at other settings of the
+    Makefile's knobs."""
+    knob = dict(k.split("=") for k in knobs)
+    in_flight = (int(knob.get("NBUF", 4)) - 1) * int(knob.get("TILE", 16)) // 4      # D tiles of TILE/4 rows per wave
+    cmd = next(l for l in subprocess.run(["make", "-n", "-B", *knobs, "_build/decode.hip.o"], cwd=PKG, check=True,
+                                         capture_output=True, text=True).stdout.split("\n") if " -c -x hip " in l)
+    args = cmd.split(" 2>&1")[0].replace("-c -x hip", "--offload-device-only -S -x hip").split()
+    asm = tmp_path / "decode.s"
+    args[args.index("-o") + 1] = str(asm)
+    subprocess.run(args, check=True, cwd=PKG, capture_output=True)
+    txt = asm.read_text()
+    for fused in (0, 1):
+        name = "_Z15lk_k_attn_splitILb%dE" % fused
+        i = txt.index("\n" + name) + 1
+        body = [l.strip() for l in txt[i:txt.index(".Lfunc_end", i)].split("\n")]
+        assert _check_paths(name, body) == (20 if fused else 4, in_flight)
+        ins = [l.split(";")[0].strip() for l in body if l and not l.startswith((";", "."))]
+        first = next(k for k, t in enumerate(ins) if t.startswith("global_load_dwordx4"))
+        wait = next(k for k, t in enumerate(ins) if k > first and "vmcnt(" in t)
+        window = ins[first:wait]
+        assert not [t for t in window if t.startswith(("s_cbranch", "s_branch")) or t.endswith(":")], (name, window)
