@@ -1327,10 +1327,10 @@ lk_k_pf_quant_rows4(const float * __restrict__ X, int ld, int kb, int8_t * __res
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int b = b0 + 32 * i;
-        float am = 0.0f;
+        float am = fabsf(x[i][0]);                            // not from 0: a block of NaN alone keeps a NaN scale
         lk_f4 t = x[i];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(x[i][e]));
+        for (int e = 1; e < 4; ++e) am = fmaxf(am, fabsf(x[i][e]));
         am = lk_max8(am);
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[e] += __shfl_xor(t[e], 4, 64);

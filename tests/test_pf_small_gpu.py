@@ -51,6 +51,40 @@ def test_quant_rows_bit_exact(lk, oracle, rows, kb, pad, offset):
     assert np.array_equal(host(sc).view(np.uint32), np.asarray(ws, np.float32).reshape(rows, kb, 2).view(np.uint32))
 
 
+def _both_forms(lk, X):
+    """The planes of X by 16-byte loads, and by single values (an address off by 4 bytes)."""
+    rows, ld = X.shape
+    out = []
+    for offset in (0, 1):
+        buf = torch.empty(rows * ld + 8, device="cuda")
+        x = buf[offset:offset + rows * ld]
+        x.copy_(dev(X.reshape(-1)))
+        qs = torch.full((rows, ld), 77, dtype=torch.int8, device="cuda")
+        sc = torch.zeros(rows, ld // 32, 2, device="cuda")
+        note(f"pf_quant_rows special values, offset={offset}")
+        lk.pf_quant_rows(x, rows, ld, ld // 32, qs, sc)
+        torch.cuda.synchronize()
+        out.append((host(qs), host(sc)))
+    return out
+
+
+# NaN and infinities: the two forms give the same bytes and scales; a block of
+# NaN alone has a NaN scale.
+def test_quant_rows_nan_and_infinite_blocks(lk):
+    rng = np.random.default_rng(5)
+    X = rng.standard_normal((6, 4 * 32)).astype(np.float32)
+    X[0, :32] = np.nan
+    X[1, 40] = np.nan
+    X[2, 64:96] = np.inf
+    X[3, 100], X[3, 101] = np.inf, -np.inf
+    X[4, :32], X[4, 7] = np.nan, np.inf
+    X[5, 32:64] = np.float32(3.4e38) * np.sign(X[5, 32:64])
+    (q4, s4), (q1, s1) = _both_forms(lk, X)
+    assert np.isnan(s1[0, 0, 0])
+    assert np.array_equal(q4, q1)
+    assert np.array_equal(s4, s1, equal_nan=True)
+
+
 # more than 8 parts per block take the wide merge: part counts off its two
 # eights, ragged last blocks, both outputs.  2e-3 of the largest output is the
 # bound every prefill case here is held to: p rounded to fp16 (2^-11 each) on
