@@ -1342,8 +1342,13 @@ lk_k_pf_quant_rows4(const float * __restrict__ X, int ld, int kb, int8_t * __res
         const float d = am / 127.0f;
         const LkQ81Div qd = lk_q81_div(am, d);
         uint32_t wq = 0;
+        if (d == 0.0f) {                                      // am up to 63 units of 2^-149: x / d is infinite
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wq |= (uint32_t) (uint8_t) lk_q81_qd(qd, x[i][e]) << (8 * e);
+            for (int e = 0; e < 4; ++e) wq |= (uint32_t) (uint8_t) lk_q81_q(x[i][e], am, d) << (8 * e);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wq |= (uint32_t) (uint8_t) lk_q81_qd(qd, x[i][e]) << (8 * e);
+        }
         if (b >= kb) continue;                                // whole 8-lane groups
         *(uint32_t *) (qs + r * kb * 32 + b * 32 + 4 * j) = wq;
         if (j == 0) sc[r * kb + b] = lk_q81_scales(d, sum);

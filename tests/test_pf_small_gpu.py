@@ -85,6 +85,20 @@ def test_quant_rows_nan_and_infinite_blocks(lk):
     assert np.array_equal(s4, s1, equal_nan=True)
 
 
+# Blocks whose maximum is a subnormal of 1 to 200 units: below 64 of them d = am /
+# 127 rounds to zero, and the quotients are infinite.
+def test_quant_rows_smallest_subnormals(lk):
+    rng = np.random.default_rng(6)
+    X = np.empty((200, 2 * 32), np.float32)
+    for r in range(200):
+        u = rng.integers(0, r + 2, 64).astype(np.uint32)
+        u[[3, 40]] = r + 1
+        X[r] = (u | (rng.integers(0, 2, 64).astype(np.uint32) << 31)).view(np.float32)
+    (q4, s4), (q1, s1) = _both_forms(lk, X)
+    assert np.array_equal(s4.view(np.uint32), s1.view(np.uint32))
+    assert np.array_equal(q4, q1)
+
+
 # more than 8 parts per block take the wide merge: part counts off its two
 # eights, ragged last blocks, both outputs.  2e-3 of the largest output is the
 # bound every prefill case here is held to: p rounded to fp16 (2^-11 each) on
