@@ -374,12 +374,13 @@ __device__ __forceinline__ void lk_pf_q81_epilogue(const lk_f4 (&a)[4], bool sto
 // a tile costs about 0.65 (0.55) of a whole one -- barrier, key scales and
 // operand reads stay -- and the workgroup beside it on the CU takes what it
 // leaves, so the plan keeps its cuts and every result its bits.  Attention and
-// merge, whole tiles -> this: 5 rows at 30000 int8 36.8 -> 26.7 us, 20 at 60000
-// 50.4 -> 37.6, 32 at 9000 22.6 -> 18.9, 77 at 30011 (Q8_1) 65.9 -> 55.7, fp16
-// 64.4 -> 51.0, 400 at 9000 (Q8_1) 71.7 -> 62.5, fp16 1100 at 3333 72.3 -> 64.3;
-// from 980 rows at 0 to 2060 at 4000 within 1% of it.  One loop with a
-// branch per pair of query blocks spilled (44-60 bytes a lane); the loops are
-// separate for that.
+// merge, whole tiles -> this, us: 5 rows at 3000 int8 19.7 -> 13.1, 5 at 30000
+// 164 -> 86.3, 20 at 4000 19.9 -> 15.2, 32 at 9000 24.1 -> 17.9, 77 at 30011
+// (Q8_1) 66.6 -> 55.0, fp16 64.1 -> 49.9, 400 at 9000 (Q8_1) 71.2 -> 60.9, 528 at
+// 20000 fp16 124 -> 104.5, 1100 at 3333 fp16 70.4 -> 62.6, 4106 at 20000 int8
+// 1203 -> 996; 980 rows at 0, int8 1100 at 3333, 2060 at 4000, 2064 and 2443 at
+// 17806 within 1% of each other.  One loop with a branch per pair of query
+// blocks spilled (44-60 bytes a lane); the loops are separate for that.
 template <bool INT8, bool PAIR, bool Q81, bool SHORT = false>
 __global__ void __launch_bounds__(PAIR ? 512 : 256, PAIR ? 1 : 2)
 lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
@@ -1073,9 +1074,22 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
                 tile(st[kt & 1], kt, nblk);
             }
         };
-        if (SHORT && m - qbase <= 16) tiles(std::integral_constant<int, 1>{});
-        else if (SHORT && m - qbase <= 32) tiles(std::integral_constant<int, 2>{});
-        else tiles(std::integral_constant<int, PF_QB>{});
+        // The order in which the loops stand decides how the compiler lays out the
+        // whole blocks' loop, which most workgroups run: 2064 rows at 17806 int8,
+        // whole blocks first / last, 473.9 / 478.8 us, 2443 425.8 / 430.8; fp16, on
+        // another run, 496.5 / 487 and 480 / 460.
+        using whole = std::integral_constant<int, PF_QB>;
+        const int rows = m - qbase;
+        if constexpr (!SHORT) tiles(whole{});
+        else if constexpr (INT8) {
+            if (rows > 32)      tiles(whole{});
+            else if (rows > 16) tiles(std::integral_constant<int, 2>{});
+            else                tiles(std::integral_constant<int, 1>{});
+        } else {
+            if (rows <= 16)      tiles(std::integral_constant<int, 1>{});
+            else if (rows <= 32) tiles(std::integral_constant<int, 2>{});
+            else                 tiles(whole{});
+        }
 
         if (pslot >= 0) {                                 // a part: unnormalised partial
             float * R = pbuf + (size_t) (pslot * LK_N_KV_HEADS + kvh) * PF_PART_SLOT;
@@ -1084,7 +1098,7 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
 #pragma unroll
             for (int qb = 0; qb < PF_QB; ++qb) {
                 const int row = 16 * qb + col;
-                if (qbase + row >= m) continue;           // never merged
+                if (SHORT && qbase + row >= m) continue;  // never merged
 #pragma unroll
                 for (int db = 0; db < 4; ++db) A[(4 * db + g) * PF_BQ + row] = acc[db][qb];
                 if (g == 0) ML[row] = make_float2(moff(qb), acc[4][qb][0]);
