@@ -1076,8 +1076,9 @@ lk_k_pf_attn(const int8_t * __restrict__ q8, const float * __restrict__ qsc,
         };
         // The order in which the loops stand decides how the compiler lays out the
         // whole blocks' loop, which most workgroups run: 2064 rows at 17806 int8,
-        // whole blocks first / last, 473.9 / 478.8 us, 2443 425.8 / 430.8; fp16, on
-        // another run, 496.5 / 487 and 480 / 460.
+        // whole blocks first / last, 473.9 / 478.8 us, 2443 425.8 / 430.8.  fp16, against
+        // a launch without short loops: last 473.0 and 441.1 (474.2 and 444.2), first,
+        // on another run, 496.5 and 479.7 (490.1 and 462.2).
         using whole = std::integral_constant<int, PF_QB>;
         const int rows = m - qbase;
         if constexpr (!SHORT) tiles(whole{});
@@ -1318,29 +1319,37 @@ lk_k_pf_combine(const float * __restrict__ pbuf, int m, int P, const PfWork work
 // Standalone planar Q8_1 of fp32 rows (reference k_pf_quant_rows,
 // prefill.cu:1574-1580), bound by HBM.  Eight lanes per 32-value block, four
 // consecutive values per lane (16-byte loads, 4-byte stores), 64 blocks per
-// workgroup as two loads per lane in flight.  The sum tree is the butterfly
+// workgroup as two loads per lane in flight: W of a row side by side, 64 / W
+// rows.  W 64 where it divides a row, else 8: 64 would leave most lanes of a
+// row of 8 blocks idle (8192 rows of 256 12.6 us, with 8 3.8), 8 always costs an
+// address per lane and load.  The sum tree is the butterfly
 // 16, 8, 4, 2, 1 over the block's values: strides 16, 8, 4 are lanes xor 4, 2,
 // 1 and strides 2, 1 the lane's own values; the quotient is formed with one
 // division per block (lk_q81_div, the same bits).  Against one value per lane
-// (4-byte loads, byte stores, a division each), in a hipGraph: 4096 rows of
-// 2048 19.7 -> 10.8 us (4.1 TB/s of 44 MB), 4096 x 8192 90.8 -> 33.0 us, 77
-// rows 2.9 -> 3.0 us (latency).  Rows whose pieces are not 16-byte aligned
-// keep the one-value form.
+// (4-byte loads, byte stores, a division each), in a hipGraph, us: 8192 rows of
+// 256 5.4 -> 3.8, 500 of 2048 3.5 -> 2.9, 4096 of 2048 18.0 -> 9.9 (44 MB), of 2304
+// 20.0 -> 10.8, of 8192 64.2 -> 30.1; 77 of 2048 2.13 -> 2.48 (latency).  Rows whose
+// pieces are not 16-byte aligned keep the one-value form.
+template <int W>
 __global__ void __launch_bounds__(256)
-lk_k_pf_quant_rows4(const float * __restrict__ X, int ld, int kb, int8_t * __restrict__ qs,
+lk_k_pf_quant_rows4(const float * __restrict__ X, int rows, int ld, int kb, int8_t * __restrict__ qs,
                     float2 * __restrict__ sc) {
 #pragma clang fp contract(off)
-    const size_t r = blockIdx.x;
-    const int j = threadIdx.x & 7, b0 = blockIdx.y * 64 + (threadIdx.x >> 3);
+    const int j = threadIdx.x & 7, u = threadIdx.x >> 3;      // load i: block u + 32i of the workgroup's 64
+    const int b0 = blockIdx.y * W;
+    const size_t r0 = (size_t) blockIdx.x * (64 / W);
     lk_f4 x[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int b = b0 + 32 * i;
-        x[i] = *(const lk_f4 *) (X + r * ld + (b < kb ? b : kb - 1) * 32 + 4 * j);   // clamped: in bounds
+        const int b = b0 + (u + 32 * i) % W;
+        const size_t r = r0 + (u + 32 * i) / W;
+        x[i] = *(const lk_f4 *) (X + (W == 64 || r < (size_t) rows ? r : rows - 1) * ld
+                                 + (b < kb ? b : kb - 1) * 32 + 4 * j);              // clamped: in bounds
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int b = b0 + 32 * i;
+        const int b = b0 + (u + 32 * i) % W;
+        const size_t r = r0 + (u + 32 * i) / W;
         float am = fabsf(x[i][0]);                            // not from 0: a block of NaN alone keeps a NaN scale
         lk_f4 t = x[i];
 #pragma unroll
@@ -1363,7 +1372,7 @@ lk_k_pf_quant_rows4(const float * __restrict__ X, int ld, int kb, int8_t * __res
 #pragma unroll
             for (int e = 0; e < 4; ++e) wq |= (uint32_t) (uint8_t) lk_q81_qd(qd, x[i][e]) << (8 * e);
         }
-        if (b >= kb) continue;                                // whole 8-lane groups
+        if (b >= kb || r >= (size_t) rows) continue;          // whole 8-lane groups
         *(uint32_t *) (qs + r * kb * 32 + b * 32 + 4 * j) = wq;
         if (j == 0) sc[r * kb + b] = lk_q81_scales(d, sum);
     }
@@ -1858,9 +1867,12 @@ extern "C" int lk_pf_quant_rows(const float * X, int rows, int ld, int kb, int8_
     if (((uintptr_t) X & 15) || ld % 4 || ((uintptr_t) qs & 3))
         hipLaunchKernelGGL(lk_k_pf_quant_rows, dim3(rows, (kb + 7) / 8), dim3(256), 0, lk_stream(stream),
                            X, ld, kb, qs, (float2 *) sc);
+    else if (kb % 64 == 0)
+        hipLaunchKernelGGL(lk_k_pf_quant_rows4<64>, dim3(rows, kb / 64), dim3(256), 0, lk_stream(stream),
+                           X, rows, ld, kb, qs, (float2 *) sc);
     else
-        hipLaunchKernelGGL(lk_k_pf_quant_rows4, dim3(rows, (kb + 63) / 64), dim3(256), 0, lk_stream(stream),
-                           X, ld, kb, qs, (float2 *) sc);
+        hipLaunchKernelGGL(lk_k_pf_quant_rows4<8>, dim3((rows - 1) / 8 + 1, (kb + 7) / 8), dim3(256), 0, lk_stream(stream),
+                           X, rows, ld, kb, qs, (float2 *) sc);
     return lk_launch_status("lk_pf_quant_rows");
 }
 
