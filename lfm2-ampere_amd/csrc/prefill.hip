@@ -1328,8 +1328,12 @@ lk_k_pf_combine(const float * __restrict__ pbuf, int m, int P, const PfWork work
 // division per block (lk_q81_div, the same bits).  Against one value per lane
 // (4-byte loads, byte stores, a division each), in a hipGraph, us: 8192 rows of
 // 256 5.4 -> 3.8, 500 of 2048 3.5 -> 2.9, 4096 of 2048 18.0 -> 9.9 (44 MB), of 2304
-// 20.0 -> 10.8, of 8192 64.2 -> 30.1; 77 of 2048 2.13 -> 2.48 (latency).  Rows whose
-// pieces are not 16-byte aligned keep the one-value form.
+// 20.0 -> 10.8, of 8192 64.2 -> 30.1.  The one-value form stays for rows whose
+// pieces are not 16-byte aligned and for launches of up to PF_Q81_FEW blocks,
+// which its shorter chain ends sooner: one value / 16 bytes, us, 77 rows of 2048
+// 2.13 / 2.48, 1000 of 256 (8000 blocks) 2.23 / 2.50, 150 of 2304 (10800) 2.45 / 2.59,
+// 250 of 2048 (16000) 2.65 / 2.58, 250 of 2304 (18000) 2.81 / 2.71.
+#define PF_Q81_FEW 14336
 template <int W>
 __global__ void __launch_bounds__(256)
 lk_k_pf_quant_rows4(const float * __restrict__ X, int rows, int ld, int kb, int8_t * __restrict__ qs,
@@ -1864,7 +1868,7 @@ extern "C" int lk_pf_quant_rows(const float * X, int rows, int ld, int kb, int8_
         return lk_fail(hipErrorInvalidValue, "lk_pf_quant_rows: rows %d, kb %d, ld %d", rows, kb, ld);
     if (rows == 0 || kb == 0) return 0;
     if (!X || !qs || !sc) return lk_fail(hipErrorInvalidValue, "lk_pf_quant_rows: null pointer argument");
-    if (((uintptr_t) X & 15) || ld % 4 || ((uintptr_t) qs & 3))
+    if ((size_t) rows * kb <= PF_Q81_FEW || ((uintptr_t) X & 15) || ld % 4 || ((uintptr_t) qs & 3))
         hipLaunchKernelGGL(lk_k_pf_quant_rows, dim3(rows, (kb + 7) / 8), dim3(256), 0, lk_stream(stream),
                            X, ld, kb, qs, (float2 *) sc);
     else if (kb % 64 == 0)

@@ -27,13 +27,14 @@ def test_kmean_bit_exact(lk, oracle, n, offset):
     assert np.array_equal(host(cm).view(np.uint32), np.asarray(want, np.float32).reshape(-1).view(np.uint32))
 
 
-# 64 blocks per workgroup, two per lane: 64 of one row, or 8 of 8 rows; ld and
-# the address decide the 16-byte path (ld % 4, offset % 4 floats); all-zero, tiny
-# and huge blocks
+# up to 14336 blocks one value per lane; above, 64 blocks per workgroup, two per
+# lane: 64 of one row, or 8 of 8 rows, where ld and the address allow 16 bytes (ld
+# % 4, offset % 4 floats); all-zero, tiny and huge blocks
 @pytest.mark.parametrize("rows,kb,pad,offset", [(1, 1, 0, 0), (3, 8, 4, 0), (5, 33, 0, 4), (2, 64, 0, 0), (3, 65, 8, 0),
                                                 (2, 130, 0, 0), (4, 64, 1, 0), (3, 9, 0, 1), (2001, 8, 0, 0),
                                                 (1600, 9, 4, 0), (447, 33, 0, 4), (225, 64, 0, 0), (113, 128, 8, 0),
-                                                (222, 65, 0, 0), (16385, 1, 0, 0), (225, 64, 1, 0), (2001, 8, 0, 1)])
+                                                (222, 65, 0, 0), (16385, 1, 0, 0), (225, 64, 1, 0), (2001, 8, 0, 1), (224, 64, 0, 0), (14336, 1, 0, 0),
+                                                (14337, 1, 0, 0)])
 def test_quant_rows_bit_exact(lk, oracle, rows, kb, pad, offset):
     rng = np.random.default_rng(rows * 1000 + kb)
     ld = kb * 32 + pad
@@ -55,7 +56,9 @@ def test_quant_rows_bit_exact(lk, oracle, rows, kb, pad, offset):
 
 
 def _both_forms(lk, X):
-    """The planes of X by 16-byte loads, and by single values (an address off by 4 bytes)."""
+    """The planes of X, repeated to more blocks than the one-value form is chosen for,
+    by 16-byte loads, and by single values (an address off by 4 bytes)."""
+    X = np.tile(X, (14336 // (X.size // 32) + 1, 1))
     rows, ld = X.shape
     out = []
     for offset in (0, 1):
