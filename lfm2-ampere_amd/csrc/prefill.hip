@@ -105,10 +105,29 @@ lk_k_pf_k8(const _Float16 * __restrict__ kc, int p0, int p1, const float * __res
 // tiles in flight, and 128 threads walk one chain each out of LDS.  Against
 // one workgroup per head whose threads load their own values (8 workgroups, a
 // memory round trip per few adds), in a hipGraph, rows read before: 1000 rows
-// 8.5 -> 5.2 us, 2999 21.5 -> 7.1, 8192 54.9 -> 9.1, 32768 593 -> 40; right
-// behind the producer that wrote 2999 rows 55 -> 6 us.
+// 7.9 -> 4.7 us, 2999 21.0 -> 6.9, 8192 54.6 -> 8.6, 32768 219 -> 27; right
+// behind the producer that wrote 2999 rows 55 -> 6 us.  Up to KM_FEW rows one
+// workgroup per head is left as it was, its memory round trips being few: 1 row
+// 1.99 us (2.11 by tiles), 77 2.08 (2.26), 128 2.41 (2.43 for 129 by tiles).
 #define KM_ROWS 1024
 #define KM_NBUF 4
+#define KM_FEW 128
+__global__ void __launch_bounds__(1024)
+lk_k_pf_kmean_few(const _Float16 * __restrict__ kc, int n, float * __restrict__ cm) {
+#pragma clang fp contract(off)
+    __shared__ float part[16][LK_HEAD_DIM];
+    const int h = blockIdx.x, d = threadIdx.x & 63, g = threadIdx.x >> 6;
+    float s = 0.0f;
+    for (int p = g; p < n; p += 16) s += (float) kc[((size_t) p * LK_N_KV_HEADS + h) * LK_HEAD_DIM + d];
+    part[g][d] = s;
+    __syncthreads();
+    if (g == 0) {
+        float t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t += part[i][d];
+        cm[h * LK_HEAD_DIM + d] = t / (float) n;
+    }
+}
 template <bool ALIGNED>                                   // kc a multiple of 16 bytes (else plain 2-byte loads)
 __global__ void __launch_bounds__(512)
 lk_k_pf_kmean(const _Float16 * __restrict__ kc, int n, float * __restrict__ cm) {
@@ -1446,7 +1465,10 @@ extern "C" int lk_pf_k8(const void * kc, int p0, int p1, const float * cm, int k
 extern "C" int lk_pf_kmean(const void * kc, int n, float * cm, void * stream) {
     if (n <= 0) return lk_fail(hipErrorInvalidValue, "lk_pf_kmean: n must be > 0");
     if (!kc || !cm) return lk_fail(hipErrorInvalidValue, "lk_pf_kmean: null pointer argument");
-    if ((uintptr_t) kc & 15)
+    if (n <= KM_FEW)
+        hipLaunchKernelGGL(lk_k_pf_kmean_few, dim3(LK_N_KV_HEADS), dim3(1024), 0, lk_stream(stream),
+                           (const _Float16 *) kc, n, cm);
+    else if ((uintptr_t) kc & 15)
         hipLaunchKernelGGL(lk_k_pf_kmean<false>, dim3(LK_N_KV_HEADS * 8), dim3(512), 0, lk_stream(stream),
                            (const _Float16 *) kc, n, cm);
     else

@@ -10,8 +10,9 @@ from gpu_util import dev, host, note
 pytestmark = pytest.mark.gpu
 
 
-# tiles of 1024 rows, four in a ring, 16 running sums: both sides of each
-@pytest.mark.parametrize("n", [1, 15, 17, 1023, 1024, 1025, 2048, 3079, 4096, 5121, 8192])
+# tiles of 1024 rows, four in a ring, 16 running sums, up to 128 rows without
+# tiles: both sides of each
+@pytest.mark.parametrize("n", [1, 15, 17, 128, 129, 145, 1023, 1024, 1025, 2048, 3079, 4096, 5121, 8192])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_kmean_bit_exact(lk, oracle, n, offset):
     rng = np.random.default_rng(n)
