@@ -36,7 +36,7 @@
 // 16 + 16 fmas, about 12 other VALU) measured 131 cycles per SIMD with 4
 // waves and everything in registers (v_fmac by DPP and v_fma_mix 4.3 cycles,
 // plain v_fma 2.7 as two waves issue together, the MFMA under them), 33 us
-// for 4096 tokens x 2048 x 2048; that launch takes 48.7-51.5 us (57-59 us in
+// for 4096 tokens x 2048 x 2048; that launch takes 51-52 us (56-59 us in
 // the form before, whose d4 took 16 bytes more of LDS reads per lane and
 // block), about 7 of them the first stage's latency and the final stores of
 // 33.5 MB.  The blocks of an output are accumulated in order, so K cannot be
@@ -116,9 +116,11 @@ __device__ __forceinline__ void pfg_fmac8(float * a, float d, const float * t) {
 }
 #undef PFG_FD
 
-// Bounded to the registers of 4 waves per SIMD although the LDS of the 128 x 64
-// shape admits 3: compiled for 3, its pipeline is ordered worse (4096 tokens
-// 51.5 -> 58.9 us).
+// Bounded to the registers of 4 waves per SIMD, which the LDS of each shape admits
+// (29, 58 and 38 KB a workgroup of 4, 16 and 4 waves, in the order of the table at
+// the launch).  128 x 64 needs 129 registers: one is spilled, before and after the
+// loop only.  Compiled for 3 waves it had the registers but an order of the pipeline
+// that was slower (4096 tokens 51.5 -> 58.9 us).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
 template <class SH, bool ADD>
@@ -210,9 +212,11 @@ lk_k_pf_gemm_q4_0(const uint8_t * __restrict__ qs, const _Float16 * __restrict__
         if (ck + 1 < nck) fetch(ck + 1);
         const uint8_t * S = stg[ck & 1];
         // The stage's NI = KC*NT MFMAs in the order block, token tile, as a
-        // pipeline: operands are read two steps ahead and the MFMA of step
+        // pipeline: operands are asked for two steps ahead and the MFMA of step
         // i + 1 is issued before the fmas of step i, so that it runs under
-        // them (the sched_barriers keep only MFMAs from moving).
+        // them (the sched_barriers keep only MFMAs from moving).  The compiler,
+        // short of registers, sinks most reads of 128 x 64 to right before their
+        // MFMA, with a wait for all of them in between.
         constexpr int NI = KC * NT;
         lk_i4g av[2], bv[2];                           // operands of the step's block / step, by parity
         uint32_t d2[2];
@@ -335,15 +339,18 @@ extern "C" int lk_pf_gemm_q4_0(const void * qs, const void * d, int N, int bpr, 
     // The shape (2048 x 2048 weights, us per launch in a hipGraph; old: the one
     // shape of 128 x 128 in 8 waves with whole-line-per-lane staging that
     // served every size before):
-    //   tokens             1    77   201   333   640  1100  1536  2048  2999  4096
-    //   old             26.4  27.8  29.7  30.9  32.2  32.6  33.3  34.7  50.7  58.9
-    //   32 x 32          6.6   7.0   8.9  11.8  16.5  27.0  32.8  41.1  57.6  75.2
-    //   128 x 128       21.6  22.5  23.5  23.3  24.1  25.8  26.6  27.7  47.6  53.5
-    //   128 x 64        16.8  17.8  18.6  18.7  19.3  27.8  27.6  29.1  40.5  51.6
-    // A launch takes a whole chain of bpr blocks per round of workgroups.  Up
-    // to 7 tiles of 32 x 32 per CU the shortest chain wins; then 128 x 128 in
-    // 16 waves while one round of the chip holds all of its tiles; past that
-    // 128 x 64, three workgroups per CU, whose rounds end less ragged.
+    //   tokens       1    77   201   333   640   896   960  1024  1100  1536  2048  2999  4096
+    //   old       25.6  27.5  29.5  30.2  30.2  30.8  30.8  30.6  31.3  32.2  33.7  49.1  56.3
+    //   32 x 32    6.3   6.6   8.0  10.0  14.6  18.7  21.5  22.2  23.9  30.6  39.9  57.1  75.7
+    //   128 x 128 21.4  22.4  22.9  23.5  23.5  23.8  23.9  24.4  24.2  24.9  28.4  48.2  53.5
+    //   128 x 64  17.0  17.9  18.0  18.3  18.3  18.9  19.2  19.1  26.7  27.0  29.3  40.5  51.4
+    // A launch takes a whole chain of bpr blocks per round of workgroups.  Up to
+    // 7 tiles of 32 x 32 per CU (256 of them) the shortest chain wins; then 128 x
+    // 128 in 16 waves while one round of the chip holds all of its tiles; past
+    // that 128 x 64, four workgroups per CU, whose rounds end less ragged.
+    // Between the first two, while the tiles of 128 x 64 fit one per CU (897 to
+    // 1024 tokens here; 1793 to 2048 for 1024 rows, 598 to 640 for 3072), 128 x 64
+    // would be shorter by 5 us: the lines do not give it that range.
     const long t32 = (long) (N / 32) * ((ntok + 31) / 32), t128 = (long) (N / 128) * ((ntok + 127) / 128);
     if (t32 <= 7 * 256)    go(PfgShape<16, 2, 2, 1, 8>{});
     else if (t128 <= 256)  go(PfgShape<32, 4, 4, 1, 4>{});
